@@ -45,6 +45,14 @@ struct PatchDev {
   uint32_t push_si[2], push_sj[2];
   CellBox recv[2];
   int32_t npush, nrecv;
+  // The cells the box kernel advances: the whole patch, or in the RK step the
+  // smallest box that holds every cell that is no exchange receiver (the
+  // exchange after the stage writes the others).  ka..kb-1 are the z positions
+  // its lanes walk (the box and one more cell on each side where there is one),
+  // npos the positions of one plane: rows of the box times kb - ka.
+  CellBox box;
+  int32_t ka, kb, npos;
+  int32_t nrecv_box;  // receive boxes that meet `box` (the first ones of recv)
 };
 
 // work item of the cell-per-thread stage kernel: patch, plane i, first (j,k) cell
@@ -1154,9 +1162,9 @@ template <typename T, bool FAST>
 __device__ __forceinline__ void add_walls(const PatchDev& P, int i, int j, int k, const T* u0, T dx, T dy, T dz,
                                           T* res) {
   const int ni = P.ni, nj = P.nj, nk = P.nk;
-  const bool wx = ni > 2 && (i == 0 || i == ni - 1);
-  const bool wy = nj > 2 && (j == 0 || j == nj - 1);
-  const bool wz = nk > 2 && (k == 0 || k == nk - 1);
+  const bool wx = ni > 2 && ((i == 0 && P.bc[0] != BC_DEAD) || (i == ni - 1 && P.bc[1] != BC_DEAD));
+  const bool wy = nj > 2 && ((j == 0 && P.bc[2] != BC_DEAD) || (j == nj - 1 && P.bc[3] != BC_DEAD));
+  const bool wz = nk > 2 && ((k == 0 && P.bc[4] != BC_DEAD) || (k == nk - 1 && P.bc[5] != BC_DEAD));
   if (!(wx || wy || wz)) return;
   const T Ax = dy * dz, Ay = dx * dz, Az = dx * dy;
   const T xc = T(0.5) * dx + T(i) * dx, yc = T(0.5) * dy + T(j) * dy, zc = T(0.5) * dz + T(k) * dz;
@@ -1197,6 +1205,362 @@ __device__ __forceinline__ void add_walls(const PatchDev& P, int i, int j, int k
 #pragma unroll
     for (int v = 0; v < 5; ++v) res[v] -= f[v];
   }
+}
+
+// ---------------------------------------------------------------------------
+// box kernel: the z-shared cell kernel over a box of each patch
+// ---------------------------------------------------------------------------
+
+// The limited slope, the face flux and its accumulation with every fusion
+// written out.  The compiler picks its own per inlined copy, and a face must
+// round alike whichever wavefront evaluates it, with boxes or without.  The
+// FP32 fast forms round as the cell-per-thread kernel (choice 11) does, bit for
+// bit: a flow that amplifies rounding, as the start of a jet, then takes the
+// same course under both.
+
+// limited() of drn_physics.h
+template <typename T, int LIM, bool FAST>
+__device__ __forceinline__ T limited_x(T d01, T d12) {
+#pragma clang fp contract(off)
+  if constexpr (LIM == LIM_VANALBADA) {
+    if constexpr (FAST) {
+      const T t = d12 * d12;
+      const T num = dfma(d12, d01, t), den = dfma(d01, d01, t) + T(1e-30);
+      return d01 * num * drcp<T, true>(den);
+    } else {
+      const T r = d12 / non_zero(d01, T(1e-10));
+      return (dfma(r, r, r) / dfma(r, r, T(1))) * d01;
+    }
+  } else {
+    return limited<T, LIM, FAST>(d01, d12);
+  }
+}
+
+// Reconstructed states of a cell u at its two faces along one axis, from its
+// neighbours m (minus side) and p (plus side); a missing neighbour is passed as
+// the cell itself with hm / hp false.  The state at the plus face is limited
+// with the minus neighbour as outer cell (upwind2.h:38-50) and the other way
+// round, so it is first order where that neighbour is missing.
+template <typename T, int RECON, int LIM, bool FAST, bool MINUS, bool PLUS>
+__device__ __forceinline__ void side_states(const T* m, const T* u, const T* p, bool hm, bool hp, T* at_minus,
+                                            T* at_plus) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int v = 0; v < 5; ++v) {
+    if constexpr (RECON != RECON_UPWIND2) {
+      if constexpr (MINUS) at_minus[v] = u[v];
+      if constexpr (PLUS) at_plus[v] = u[v];
+    } else if constexpr (FAST && (LIM == LIM_VANALBADA || LIM == LIM_MINMOD)) {
+      // symmetric limited slope: one for both faces, and exactly zero when a
+      // neighbour is the cell itself (one difference is zero)
+      const T s = limited_x<T, LIM, true>(u[v] - m[v], p[v] - u[v]);
+      if constexpr (MINUS) at_minus[v] = dfma(T(-0.5), s, u[v]);
+      if constexpr (PLUS) at_plus[v] = dfma(T(0.5), s, u[v]);
+    } else {
+      if constexpr (MINUS) {
+        const T s = limited_x<T, LIM, FAST>(u[v] - p[v], m[v] - u[v]);
+        at_minus[v] = hp ? dfma(T(0.5), s, u[v]) : u[v];
+      }
+      if constexpr (PLUS) {
+        const T s = limited_x<T, LIM, FAST>(u[v] - m[v], p[v] - u[v]);
+        at_plus[v] = hm ? dfma(T(0.5), s, u[v]) : u[v];
+      }
+    }
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void load5(const char* const* sv, uint32_t off, T* u) {
+#pragma unroll
+  for (int v = 0; v < 5; ++v) u[v] = ldv<T>(sv[v], off);
+}
+template <typename T>
+__device__ __forceinline__ void add5(T* res, const T* f) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int v = 0; v < 5; ++v) res[v] += f[v];
+}
+template <typename T>
+__device__ __forceinline__ void sub5(T* res, const T* f) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int v = 0; v < 5; ++v) res[v] -= f[v];
+}
+
+// One face's AUSM+ flux along DIR as sums of products: density x * y, momentum
+// and energy c fl * l[c] + fr * r[c], and pa * ps more for the normal momentum.
+template <typename T>
+struct FaceFlux {
+  T x, y, fl, fr, l[4], r[4], pa, ps;
+  // the flux itself
+  template <int DIR>
+  __device__ __forceinline__ void set(T* f) const {
+#pragma clang fp contract(off)
+    f[0] = x * y;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      f[1 + c] = dfma(fl, l[c], fr * r[c]);
+      if (c == DIR) f[1 + c] = dfma(pa, ps, f[1 + c]);
+    }
+  }
+  // the flux f (from set) added to res, the density product in one rounding
+  __device__ __forceinline__ void add(const T* f, T* res) const {
+#pragma clang fp contract(off)
+    res[0] = dfma(x, y, res[0]);
+#pragma unroll
+    for (int v = 1; v < 5; ++v) res[v] += f[v];
+  }
+};
+
+// M4(M, S) and P5(M, S) of M = un * ia for S = +1 or -1 (mach_split_fast of
+// drn_physics.h); M + S, M - S and 2 S - M take the product unrounded
+template <typename T, int S>
+__device__ __forceinline__ void mach_split_x(T un, T ia, T& m4, T& p5) {
+#pragma clang fp contract(off)
+  const T M = un * ia;
+  const T t1 = dfma(un, ia, T(S)), t2 = dfma(un, ia, T(-S));
+  const T q2 = t2 * t2;
+  const T m2 = T(0.25 * S) * (t1 * t1);
+  const T m4p = m2 * dfma(T(0.5), q2, T(1));
+  const T p5p = m2 * dfma(T(0.75) * M, q2, dfma(-un, ia, T(2 * S)));
+  const bool sup = dabs(M) >= T(1);
+  const T m1 = S > 0 ? (M > T(0) ? M : T(0)) : (M < T(0) ? M : T(0));
+  const T p1 = T(S) * M > T(0) ? T(1) : T(0);
+  m4 = sup ? m1 : m4p;
+  p5 = sup ? p1 : p5p;
+}
+
+template <typename T, bool FAST, int DIR>
+__device__ __forceinline__ FaceFlux<T> face_flux_x(const T* vl, const T* vr, T A) {
+#pragma clang fp contract(off)
+  FaceFlux<T> F;
+  T m4l, p5l, m4r, p5r;
+  if constexpr (FAST) {
+    const PrimFast<T> L = lr_vars_fast(vl), R = lr_vars_fast(vr);
+    const T unl = DIR == 0 ? L.u : (DIR == 1 ? L.v : L.w);
+    const T unr = DIR == 0 ? R.u : (DIR == 1 ? R.v : R.w);
+    const T a = T(0.5) * (L.a + R.a);
+    const T ia = drcp<T, true>(a);
+    mach_split_x<T, 1>(unl, ia, m4l, p5l);
+    mach_split_x<T, -1>(unr, ia, m4r, p5r);
+    const T M = m4l + m4r;
+    const T Mp = M > T(0) ? M : T(0), Mm = M < T(0) ? M : T(0);
+    F.x = a * A;
+    F.y = dfma(L.r, Mp, R.r * Mm);
+    const T f0 = F.x * F.y;
+    F.fl = f0 > T(0) ? f0 : T(0);
+    F.fr = f0 < T(0) ? f0 : T(0);
+    F.l[0] = L.u, F.l[1] = L.v, F.l[2] = L.w, F.l[3] = L.H;
+    F.r[0] = R.u, F.r[1] = R.v, F.r[2] = R.w, F.r[3] = R.H;
+    F.pa = A * (Gas<T>::R / Gas<T>::CV);
+    F.ps = dfma(p5l, L.re, p5r * R.re);
+  } else {
+    T rl, rr, al, ar, pl, pr;
+    auto prim = [](const T* var, T& r, T& a, T& p, T* q) {
+      r = var[0];
+      const T ir = T(1) / r;
+      q[0] = var[1] * ir, q[1] = var[2] * ir, q[2] = var[3] * ir;
+      // rounded as the slip wall's: a row uniform across a wall stays uniform
+      const T e = dfma(var[4], ir, T(-0.5) * dfma(q[2], q[2], dfma(q[0], q[0], q[1] * q[1])));
+      const T Tt = e / Gas<T>::CV;
+      p = r * Gas<T>::R * Tt;
+      a = dsqrt(Gas<T>::GAMMA * Gas<T>::R * Tt);
+      q[3] = (var[4] + p) / r;
+    };
+    prim(vl, rl, al, pl, F.l);
+    prim(vr, rr, ar, pr, F.r);
+    const T a = T(0.5) * (al + ar);
+    mach_split_x<T, 1>(F.l[DIR] / a, T(1), m4l, p5l);
+    mach_split_x<T, -1>(F.r[DIR] / a, T(1), m4r, p5r);
+    const T M = m4l + m4r;
+    F.x = a * A;
+    F.y = dfma(rl, M > T(0) ? M : T(0), rr * (M < T(0) ? M : T(0)));
+    const T f0 = F.x * F.y;
+    F.fl = f0 > T(0) ? f0 : T(0);
+    F.fr = f0 < T(0) ? f0 : T(0);
+    F.pa = A;
+    F.ps = dfma(p5l, pl, p5r * pr);
+  }
+  return F;
+}
+
+// One thread per cell of the patch's box (PatchDev::box; in the RK step the
+// cells that are no exchange receivers).  A wavefront walks 62 consecutive
+// positions of the plane's flattened (row, k) space; lanes 0 and 63 hold the
+// next positions on either side, so that every z slope is formed by one lane
+// only and a z face by one lane only (the state at the face comes from the lane
+// below, the face flux goes back to it).  A row's positions are the z range of
+// the box and one cell beyond it on each side, so a row end needs no other
+// lane.  XP = 4: the item's four wavefronts cover four planes at the same
+// positions; those above the first take their x face i-1/2 from the wavefront
+// below through LDS (one barrier; the y neighbours are loaded before it).
+//   face evaluations per cell: x 2 (XP = 4: 1.25), y 2, z 1
+//   limited slopes per cell:   x 3 (XP = 4: 2.25), y 3, z 1
+// against 4.52 and 7.5 of k_stage_cell_xs<2> (FP32 fast arithmetic; the other
+// forms take two limited states per slope there and here).  68 VGPRs in FP32.
+// What bounds it: on a 64-patch jet of 19.2 M cells (state buffers beyond the
+// caches) the same loads and stores without the fluxes take 0.42 ms of its 0.47
+// ms per stage, on a grid that the caches hold 52 of 78 us: the five planes and
+// five rows of the stencil come from L2 and share its path with the state's own
+// traffic.  Four planes per item read least through it.
+template <typename T, int RECON, int LIM, bool FAST, int XP>
+__device__ __forceinline__ void stage_box_item(const PatchDev* __restrict__ pds, const TileCell t,
+                                               const T* __restrict__ src, const T* base, T* dst, uint64_t vs,
+                                               T factor, int push, T* xbuf) {
+  const PatchDev& P = pds[t.patch];
+  const int ni = P.ni, nj = P.nj, nk = P.nk, njk = P.njk;
+  const int lane = (int)(threadIdx.x & 63);
+  constexpr int WPP = 4 / XP;  // wavefronts per plane
+  // the wavefront's number as a scalar: its plane and the tests on it are scalar too
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), pw = wv / WPP;
+  const int i = t.i + pw;
+  const int ii = i < P.box.i1 ? i : P.box.i1 - 1;  // a plane of the box for the addresses
+  const int q = t.c2 + 62 * (wv % WPP) + lane - 1;
+  const int pitch = P.kb - P.ka;
+  const int qq = q < 0 ? 0 : (q < P.npos ? q : P.npos - 1);
+  const int jr = qq / pitch;
+  const int j = P.box.j0 + jr, k = P.ka + qq - jr * pitch;
+  const bool in = q >= 0 && q < P.npos && (XP == 1 || i < P.box.i1);
+  const bool own = in && lane >= 1 && lane <= 62 && k >= P.box.k0 && k < P.box.k1;
+  constexpr uint32_t W = sizeof(T);
+  const uint32_t sx = (uint32_t)njk * W, sy = (uint32_t)nk * W;
+  const uint32_t c = (P.off + (uint32_t)ii * (uint32_t)njk + (uint32_t)j * (uint32_t)nk + (uint32_t)k) * W;
+  const char* sv[5];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) sv[v] = reinterpret_cast<const char*>(src + (uint64_t)v * vs);
+  const T dx = T(P.dx), dy = T(P.dy), dz = T(P.dz);
+  const T Ax = dy * dz, Ay = dx * dz, Az = dx * dy;
+  T u[5], res[5], fxp[5], fyp[5], none[5];
+  load5<T>(sv, c, u);
+  zero5(res);
+  zero5(fxp);
+  zero5(fyp);
+  // Residual in the reference's order Fx- + Fy- + Fz- - Fz+ - Fy+ - Fx+
+  if (ni > 2 && own) {
+    const uint32_t m1 = ii >= 1 ? sx : 0u, m2 = ii >= 2 ? 2 * sx : m1;
+    const uint32_t p1 = ii + 1 < ni ? sx : 0u, p2 = ii + 2 < ni ? 2 * sx : p1;
+    T um[5], up[5], lo[5], hi[5], o[5];
+    load5<T>(sv, c - m1, um);
+    load5<T>(sv, c + p1, up);
+    side_states<T, RECON, LIM, FAST, true, true>(um, u, up, ii >= 1, ii + 1 < ni, lo, hi);
+    if (ii > 0 && pw == 0) {
+      T umm[5];
+      load5<T>(sv, c - m2, umm);
+      side_states<T, RECON, LIM, FAST, false, true>(umm, um, u, ii >= 2, true, none, o);
+      face_flux_x<T, FAST, 0>(o, lo, Ax).template set<0>(res);
+    }
+    if (ii + 1 < ni) {
+      T upp[5];
+      load5<T>(sv, c + p2, upp);
+      side_states<T, RECON, LIM, FAST, true, false>(u, up, upp, true, ii + 2 < ni, o, none);
+      face_flux_x<T, FAST, 0>(hi, o, Ax).template set<0>(fxp);
+    }
+    if constexpr (XP > 1) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) xbuf[(wv * 5 + v) * 64 + lane] = fxp[v];
+    }
+  }
+  // the rows around, a missing one replaced by the nearest row
+  T ym2[5], ym1[5], yp1[5], yp2[5];
+  const bool hy_m = j >= 1, hy_p = j + 1 < nj;
+  if (own) {
+    const uint32_t om1 = hy_m ? c - sy : c, om2 = j >= 2 ? om1 - sy : om1;
+    const uint32_t op1 = hy_p ? c + sy : c, op2 = j + 2 < nj ? op1 + sy : op1;
+    load5<T>(sv, om2, ym2);
+    load5<T>(sv, om1, ym1);
+    load5<T>(sv, op1, yp1);
+    load5<T>(sv, op2, yp2);
+  }
+  if constexpr (XP > 1) {
+    __syncthreads();
+    if (pw > 0 && ii > 0 && ni > 2 && own) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) res[v] = xbuf[((wv - WPP) * 5 + v) * 64 + lane];
+    }
+  }
+  if (nj > 2 && own) {
+    T lo[5], hi[5], o[5];
+    side_states<T, RECON, LIM, FAST, true, true>(ym1, u, yp1, hy_m, hy_p, lo, hi);
+    if (hy_m) {
+      side_states<T, RECON, LIM, FAST, false, true>(ym2, ym1, u, j >= 2, true, none, o);
+      const FaceFlux<T> F = face_flux_x<T, FAST, 1>(o, lo, Ay);
+      T f[5];
+      F.template set<1>(f);
+      F.add(f, res);
+    }
+    if (hy_p) {
+      side_states<T, RECON, LIM, FAST, true, false>(u, yp1, yp2, true, j + 2 < nj, o, none);
+      face_flux_x<T, FAST, 1>(hi, o, Ay).template set<1>(fyp);
+    }
+  }
+  // z: the neighbours are the next lanes' cells; at a row end and at the
+  // wavefront's ends the lane loads the cell outside (the cell itself stands in
+  // at the patch ends)
+  if (nk > 2) {
+    const bool hz_m = k >= 1, hz_p = k + 1 < nk;
+    T um[5], up[5], lo[5], hi[5], f[5], o[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      um[v] = __shfl_up(u[v], 1, 64);
+      up[v] = __shfl_down(u[v], 1, 64);
+    }
+    if (in && hz_m && (lane == 0 || k == P.ka)) load5<T>(sv, c - W, um);
+    if (in && hz_p && (lane == 63 || k + 1 == P.kb)) load5<T>(sv, c + W, up);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      if (!hz_m) um[v] = u[v];
+      if (!hz_p) up[v] = u[v];
+    }
+    side_states<T, RECON, LIM, FAST, true, true>(um, u, up, hz_m, hz_p, lo, hi);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) o[v] = __shfl_up(hi[v], 1, 64);
+    zero5(f);
+    if (in && k > P.ka) {
+      const FaceFlux<T> F = face_flux_x<T, FAST, 2>(o, lo, Az);
+      F.template set<2>(f);
+      F.add(f, res);
+    }
+    // the plus face: the next position's minus face, zero where a row ends
+#pragma unroll
+    for (int v = 0; v < 5; ++v) o[v] = __shfl_down(f[v], 1, 64);
+    sub5(res, o);
+  }
+  sub5(res, fyp);
+  sub5(res, fxp);
+  if (!own) return;
+  // patch-face functors (cartesianiterator.h:190-308)
+  add_walls<T, FAST>(P, i, j, k, u, dx, dy, dz, res);
+  // cartesianiterator.h:310-322
+  const T pf = factor / (dx * dy * dz);
+  T nv[5];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) nv[v] = ldv<T>(reinterpret_cast<const char*>(base + (uint64_t)v * vs), c) + pf * res[v];
+  bool store = true;
+  if (push) {
+    // the fused exchange of the z-face seek layers, as in stage_cell_item
+    for (int s = 0; s < P.nrecv_box; ++s) store = store && !in_box(P.recv[s], i, j, k);
+    for (int s = 0; s < P.npush; ++s) {
+      if (in_box(P.push[s], i, j, k)) {
+        const uint32_t tb =
+            ((uint32_t)P.push_base[s] + (uint32_t)i * P.push_si[s] + (uint32_t)j * P.push_sj[s] + (uint32_t)k) * W;
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+          *reinterpret_cast<T*>(reinterpret_cast<char*>(dst + (uint64_t)v * vs) + tb) = T(0) + nv[v];
+      }
+    }
+  }
+  if (store) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) *reinterpret_cast<T*>(reinterpret_cast<char*>(dst + (uint64_t)v * vs) + c) = nv[v];
+  }
+}
+
+template <typename T, int RECON, int LIM, bool FAST, int XP>
+__global__ __launch_bounds__(256) void k_stage_box(const PatchDev* __restrict__ pds, const TileCell* __restrict__ tiles,
+                                                   const T* __restrict__ src, const T* base, T* dst, uint64_t vs,
+                                                   T factor, int push) {
+  __shared__ T xbuf[XP > 1 ? 4 * 5 * 64 : 1];
+  stage_box_item<T, RECON, LIM, FAST, XP>(pds, tiles[blockIdx.x], src, base, dst, vs, factor, push, xbuf);
 }
 
 // One thread per column of two cells (i0, i0+1): the x face between them is

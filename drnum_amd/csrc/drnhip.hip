@@ -99,6 +99,14 @@ struct drn_ctx {
     std::vector<int> first;
     TileCell *d = nullptr, *d_xcd = nullptr, *d_xcd_pp = nullptr, *d_chain = nullptr;
   } xs[2];
+  // items of the box kernel over the boxes of the patch descriptors: [0] one
+  // plane, [1] four planes per item; `box` covers whole patches, `box_rk` the
+  // boxes of the RK step's descriptors (empty where those are not set)
+  struct BoxList {
+    int n = 0;               // items of the batched list
+    std::vector<int> first;  // per patch, size np+1 (into d_pp)
+    TileCell *d = nullptr, *d_pp = nullptr;  // both in XCD segments
+  } box[2], box_rk[2];
   std::vector<TileCell> tx2;
   std::vector<int> tx2_first;
   TileCell* d_tx2 = nullptr;
@@ -114,8 +122,8 @@ struct drn_ctx {
   double* d_out = nullptr;
   void* d_post = nullptr;    // post-processing output of one patch
   size_t post_bytes = 0;
-  int tiling = 11;     // batched form
-  int tiling_pp = 11;  // per-patch form
+  int tiling = -1;     // batched form; -1: by auto_tiling until one is set
+  int tiling_pp = -1;  // per-patch form
   int arith = -1;  // DRN_ARITH_*; -1 = precision default
   // marching work-lists: batched (launch order) and per-patch (natural order, patch-contiguous)
   std::vector<TileMarch> mt_pp;
@@ -271,7 +279,9 @@ enum {
   K_XM7 = 11,    // K_XM capped at 7 waves per SIMD (FP32 fast arithmetic; else K_XM)
   K_XML = 12,    // K_XM with the x slope and x face flux carried in LDS
   K_CELLXS2 = 13,  // the z-shared cell kernel over 2 planes per item, x faces shared through LDS
-  K_CELLXS4 = 14   // the same over 4 planes per item
+  K_CELLXS4 = 14,  // the same over 4 planes per item
+  K_BOX1 = 15,     // one thread per cell of the patch's box, one plane per item
+  K_BOX4 = 16      // the same over 4 planes per item, x faces shared through LDS
 };
 struct TilingChoice {
   int irange;  // planes per work item, 0 = whole patch
@@ -291,8 +301,9 @@ static const TilingChoice kTilings[] = {
     {0, 2, K_CELLZ},   {0, 1, K_XM},         {32, 1, K_XM},    {16, 1, K_XM},    {8, 1, K_XM},
     {0, 1, K_XM8},     {16, 1, K_XM8},       {0, 1, K_XM7},    {16, 1, K_XM7},   {0, 1, K_XML},
     {16, 1, K_XML},    {8, 1, K_XML},        {0, 2, K_CELLXS4}, {0, 1, K_CELLXS4}, {0, 2, K_CELLXS2},
-    {0, 1, K_CELLXS2}};
+    {0, 1, K_CELLXS2}, {0, 2, K_BOX1},      {0, 2, K_BOX4}};
 static const int kNumTilings = sizeof(kTilings) / sizeof(kTilings[0]);
+static const int kBoxOnePlane = 51, kBoxFourPlanes = 52;
 
 // the column kernel covers the fast MUSCL forms with a symmetric limited slope
 static bool column_capable(const drn_ctx* ctx);
@@ -354,7 +365,13 @@ static void launch_range(drn_ctx* ctx, int kind, const void* tiles, int ntiles, 
                                        kind == K_CELL_SLOPE);
   else if (kind == K_WTILE)
     launch_wtile_t<T, RECON, LIM, FAST>(ctx, (const TileWave*)tiles, ntiles, src, base, dst, factor);
-  else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
+  else if (kind == K_BOX1 || kind == K_BOX4) {
+    if (ntiles > 0) {
+      const auto kern = kind == K_BOX1 ? k_stage_box<T, RECON, LIM, FAST, 1> : k_stage_box<T, RECON, LIM, FAST, 4>;
+      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, ctx->stream, ctx->pd_stage, (const TileCell*)tiles, src, base,
+                         dst, ctx->vstride, factor, (int)ctx->push_now);
+    }
+  } else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
     if (ntiles > 0) {
       if (kind == K_CELLXS2)
         hipLaunchKernelGGL((k_stage_cell_xs<T, RECON, LIM, FAST, 2>), dim3(ntiles), dim3(256), 0, ctx->stream,
@@ -450,6 +467,22 @@ static bool column_capable(const drn_ctx* ctx) {
   return fast && ctx->recon == DRN_RECON_UPWIND2 && (ctx->lim == DRN_LIM_VANALBADA || ctx->lim == DRN_LIM_MINMOD);
 }
 
+// The tiling choice of a launch form: the one set or autotuned, else by a rule.
+// The box kernel over four planes per item (52) is the fastest or within 6 % of
+// it on every grid measured from 0.3 to 60 M cells in both precisions (64-patch
+// jet, FP32: 0.467 ms per stage and exchange against 0.612 of choice 11 and
+// 0.495 of 49; 27-patch jet, FP64: 0.303 against 0.458 and 0.351 of 48).  Where
+// its items would not give every CU one, the one-plane form (51) spreads the
+// cells over four times as many workgroups: 8 patches of 8^3 cells, FP64, 14.2
+// us against 22.7; 8 patches of 16^3, FP32, 160 items, 9.4 against 9.5.
+static int tiling_of(const drn_ctx* ctx, int launch) {
+  const int set = launch == DRN_LAUNCH_BATCHED ? ctx->tiling : ctx->tiling_pp;
+  if (set >= 0) return set;
+  const int n = (ctx->box_rk[1].n > 0 ? ctx->box_rk : ctx->box)[1].n;
+  const int np = launch == DRN_LAUNCH_BATCHED ? 1 : std::max(1, (int)ctx->descs.size());
+  return n / np < ctx->n_cu ? kBoxOnePlane : kBoxFourPlanes;
+}
+
 // effective kernel kind of a tiling choice in the current arithmetic/operator;
 // with the viscous flux every choice runs the z-shared cell kernel on its list
 // order (the other kernels carry the Euler flux only)
@@ -467,6 +500,11 @@ static bool fast_math(const drn_ctx* ctx) {
   return ctx->arith < 0 ? ctx->prec == DRN_F32 : ctx->arith == DRN_ARITH_FAST;
 }
 
+// the box kernel's items over the boxes of the descriptors of this stage
+static const drn_ctx::BoxList& box_list(const drn_ctx* ctx, int kind) {
+  return (ctx->pd_stage == ctx->d_pd ? ctx->box : ctx->box_rk)[kind == K_BOX4 ? 1 : 0];
+}
+
 template <typename T>
 static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int launch) {
   const T* src = (const T*)ctx->buf[psrc];
@@ -479,22 +517,25 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
     else
       launch_dispatch<T, false>(ctx, kind, tl, n, src, base, dst, factor);
   };
+  const int choice = tiling_of(ctx, launch), kind = effective_kind(ctx, choice);
   if (launch == DRN_LAUNCH_BATCHED) {
-    const int kind = effective_kind(ctx, ctx->tiling);
-    if (kind == K_CELLXS2 || kind == K_CELLXS4) {
+    if (kind == K_BOX1 || kind == K_BOX4) {
+      const auto& L = box_list(ctx, kind);
+      go(kind, L.d, L.n);
+    } else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
       const auto& L = ctx->xs[kind == K_CELLXS4 ? 1 : 0];
-      const int xo = kTilings[ctx->tiling].xcd;
+      const int xo = kTilings[choice].xcd;
       go(kind, xo == 2 && L.d_chain ? L.d_chain : (xo ? L.d_xcd : L.d), (int)L.nat.size());
     } else if (kind == K_CELLX2) {
-      go(K_CELLX2, kTilings[ctx->tiling].xcd ? ctx->d_tx2_xcd : ctx->d_tx2, (int)ctx->tx2.size());
+      go(K_CELLX2, kTilings[choice].xcd ? ctx->d_tx2_xcd : ctx->d_tx2, (int)ctx->tx2.size());
     } else if (kind == K_CELLYZ) {
-      go(K_CELLYZ, kTilings[ctx->tiling].xcd ? ctx->d_tyz_xcd : ctx->d_tyz, (int)ctx->tyz.size());
+      go(K_CELLYZ, kTilings[choice].xcd ? ctx->d_tyz_xcd : ctx->d_tyz, (int)ctx->tyz.size());
     } else if (kind == K_CELLZ || kind == K_CELLZP) {
-      const int xo = kTilings[ctx->tiling].xcd;
+      const int xo = kTilings[choice].xcd;
       const TileCell* tl = xo == 2 && ctx->d_tz_chain ? ctx->d_tz_chain : (xo ? ctx->d_tz_xcd : ctx->d_tz);
       go(kind, tl, (int)ctx->tz.size());
     } else if (kind == K_CELL || kind == K_CELL_SLOPE) {
-      go(kind, kTilings[ctx->tiling].xcd ? ctx->d_tiles_xcd : ctx->d_tiles, (int)ctx->tiles.size());
+      go(kind, kTilings[choice].xcd ? ctx->d_tiles_xcd : ctx->d_tiles, (int)ctx->tiles.size());
     } else if (kind == K_WTILE) {
       go(K_WTILE, ctx->d_wt_launch, ctx->n_wt);
       go(K_CELL, ctx->d_thin_tiles, (int)ctx->thin_tiles.size());
@@ -503,32 +544,34 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
       go(K_CELL, ctx->d_thin_tiles, (int)ctx->thin_tiles.size());
     }
   } else {
-    const int kind = effective_kind(ctx, ctx->tiling_pp);
     const int np = (int)ctx->descs.size();
     for (int p = 0; p < np; ++p) {
       const int m0 = ctx->mt_first[p], mn = ctx->mt_first[p + 1] - m0;
       const int w0 = ctx->wt_first[p], wn = ctx->wt_first[p + 1] - w0;
-      if (kind == K_CELLXS2 || kind == K_CELLXS4) {
+      if (kind == K_BOX1 || kind == K_BOX4) {
+        const auto& L = box_list(ctx, kind);
+        go(kind, L.d_pp + L.first[p], L.first[p + 1] - L.first[p]);
+      } else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
         const auto& L = ctx->xs[kind == K_CELLXS4 ? 1 : 0];
         const int z0 = L.first[p];
-        go(kind, (kTilings[ctx->tiling_pp].xcd ? L.d_xcd_pp : L.d) + z0, L.first[p + 1] - z0);
+        go(kind, (kTilings[choice].xcd ? L.d_xcd_pp : L.d) + z0, L.first[p + 1] - z0);
       } else if (kind == K_CELLX2) {
         const int z0 = ctx->tx2_first[p];
-        const TileCell* tl = (kTilings[ctx->tiling_pp].xcd ? ctx->d_tx2_xcd_pp : ctx->d_tx2) + z0;
+        const TileCell* tl = (kTilings[choice].xcd ? ctx->d_tx2_xcd_pp : ctx->d_tx2) + z0;
         go(K_CELLX2, tl, ctx->tx2_first[p + 1] - z0);
       } else if (kind == K_CELLYZ) {
         const int z0 = ctx->tyz_first[p];
-        const TileCell* tl = (kTilings[ctx->tiling_pp].xcd ? ctx->d_tyz_xcd_pp : ctx->d_tyz) + z0;
+        const TileCell* tl = (kTilings[choice].xcd ? ctx->d_tyz_xcd_pp : ctx->d_tyz) + z0;
         go(K_CELLYZ, tl, ctx->tyz_first[p + 1] - z0);
       } else if (kind == K_CELLZ || kind == K_CELLZP) {
         const int z0 = ctx->tz_first[p];
-        const TileCell* tl = (kTilings[ctx->tiling_pp].xcd ? ctx->d_tz_xcd_pp : ctx->d_tz) + z0;
+        const TileCell* tl = (kTilings[choice].xcd ? ctx->d_tz_xcd_pp : ctx->d_tz) + z0;
         go(kind, tl, ctx->tz_first[p + 1] - z0);
       } else if (kind == K_WTILE && wn > 0) {
         go(K_WTILE, ctx->d_wt_pp + w0, wn);
       } else if (kind == K_CELL || kind == K_CELL_SLOPE || kind == K_WTILE || mn == 0) {
         const int t0 = ctx->tile_first[p];
-        const TileCell* tl = (kTilings[ctx->tiling_pp].xcd ? ctx->d_tiles_xcd_pp : ctx->d_tiles) + t0;
+        const TileCell* tl = (kTilings[choice].xcd ? ctx->d_tiles_xcd_pp : ctx->d_tiles) + t0;
         go(kind == K_CELL_SLOPE ? K_CELL_SLOPE : K_CELL, tl, ctx->tile_first[p + 1] - t0);
       } else {
         go(kind, ctx->d_mt_pp + m0, mn);
@@ -541,14 +584,14 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
 // fused z-face receivers themselves; the other kinds leave them to the exchange.
 static bool push_kind(int kind) {
   return kind == K_CELL || kind == K_CELLZ || kind == K_CELLZP || kind == K_XM || kind == K_XM8 || kind == K_XM7 ||
-         kind == K_XML || kind == K_CELLXS2 || kind == K_CELLXS4;
+         kind == K_XML || kind == K_CELLXS2 || kind == K_CELLXS4 || kind == K_BOX1 || kind == K_BOX4;
 }
 
 // whether a stage of this launch form fills the fused receivers (and the
 // exchange after it then runs on the lists without them)
 static bool push_active(const drn_ctx* ctx, int launch) {
   if (!ctx->fuse || !ctx->have_exchange || ctx->n_fused == 0) return false;
-  return push_kind(effective_kind(ctx, launch == DRN_LAUNCH_BATCHED ? ctx->tiling : ctx->tiling_pp));
+  return push_kind(effective_kind(ctx, tiling_of(ctx, launch)));
 }
 
 // rk: a stage of the RK step (or the autotuner's stand-in for one), whose
@@ -598,7 +641,8 @@ static int chunk_of(const drn_ctx* ctx, int choice) {
 
 // build the marching work-lists of the current tiling choices of both launch forms
 static int build_march(drn_ctx* ctx) {
-  const TilingChoice tb = kTilings[ctx->tiling], tp = kTilings[ctx->tiling_pp];
+  const int cb = tiling_of(ctx, DRN_LAUNCH_BATCHED), cp = tiling_of(ctx, DRN_LAUNCH_PER_PATCH);
+  const TilingChoice tb = kTilings[cb], tp = kTilings[cp];
   const int np = (int)ctx->descs.size();
   std::vector<TileMarch> nat;
   std::vector<TileWave> wnat;
@@ -635,8 +679,8 @@ static int build_march(drn_ctx* ctx) {
     lf = std::max(lf, plf);
     lsy = std::max(lsy, psy);
     lsz = std::max(lsz, psz);
-    march_items(d, p, tb.irange, chunk_of(ctx, ctx->tiling), nat);
-    march_items(d, p, tp.irange, chunk_of(ctx, ctx->tiling_pp), ctx->mt_pp);
+    march_items(d, p, tb.irange, chunk_of(ctx, cb), nat);
+    march_items(d, p, tp.irange, chunk_of(ctx, cp), ctx->mt_pp);
     ctx->wt_first[p] = (int)ctx->wt_pp.size();
     if (tb.kind == K_WTILE) wtile_items(d, p, tb.irange, wnat);
     if (tp.kind == K_WTILE) wtile_items(d, p, tp.irange, ctx->wt_pp);
@@ -698,6 +742,71 @@ static int build_march(drn_ctx* ctx) {
   if (!ctx->thin_tiles.empty())
     HIPCHK(ctx, hipMemcpy(ctx->d_thin_tiles, ctx->thin_tiles.data(), ctx->thin_tiles.size() * sizeof(TileCell),
                           hipMemcpyHostToDevice));
+  return DRN_OK;
+}
+
+// the descriptor's fields of the box kernel for the box [i0,i1) x [j0,j1) x [k0,k1)
+static void set_box(PatchDev& P, const CellBox& b) {
+  P.box = b;
+  P.ka = std::max(0, b.k0 - 1);
+  P.kb = std::min(P.nk, b.k1 + 1);
+  P.npos = (b.j1 - b.j0) * (P.kb - P.ka);
+}
+
+static void free_box(drn_ctx::BoxList& L) {
+  dfree(L.d);
+  dfree(L.d_pp);
+  L.d = L.d_pp = nullptr;
+  L.n = 0;
+  L.first.clear();
+}
+
+// The box kernel's work lists (both plane counts) over the boxes of `pd`: the
+// planes of a chain's patches side by side, then in 8 contiguous segments, one
+// per XCD; and per patch.  An item covers 62 positions per wavefront.
+static int build_box(drn_ctx* ctx, const std::vector<PatchDev>& pd, const std::vector<std::vector<int>>& chains,
+                      drn_ctx::BoxList* lists) {
+  auto segment = [](const std::vector<TileCell>& nat, size_t a, size_t b, std::vector<TileCell>& out) {
+    const size_t n = b - a, seg = (n + 7) / 8;
+    for (size_t r = 0; r < seg; ++r)
+      for (size_t x = 0; x < 8; ++x)
+        if (x * seg + r < n) out.push_back(nat[a + x * seg + r]);
+  };
+  const int np = (int)pd.size();
+  for (int w = 0; w < 2; ++w) {
+    drn_ctx::BoxList& L = lists[w];
+    free_box(L);
+    const int xp = w == 1 ? 4 : 1, step = 62 * 4 / xp;
+    auto plane = [&](int p, int i, std::vector<TileCell>& out) {
+      for (int c2 = 0; c2 < pd[p].npos; c2 += step) out.push_back(TileCell{p, i, c2, 0});
+    };
+    std::vector<TileCell> nat, all, pp;
+    for (const auto& ch : chains) {
+      int lo = 32767, hi = 0;
+      for (int p : ch) {
+        lo = std::min(lo, pd[p].box.i0);
+        hi = std::max(hi, pd[p].box.i1);
+      }
+      for (int i = lo; i < hi; ++i)
+        for (int p : ch)
+          if (i >= pd[p].box.i0 && i < pd[p].box.i1 && (i - pd[p].box.i0) % xp == 0) plane(p, i, nat);
+    }
+    segment(nat, 0, nat.size(), all);
+    L.n = (int)all.size();
+    L.first.assign(np + 1, 0);
+    nat.clear();
+    for (int p = 0; p < np; ++p) {
+      const size_t a = nat.size();
+      L.first[p] = (int)a;
+      for (int i = pd[p].box.i0; i < pd[p].box.i1; i += xp) plane(p, i, nat);
+      segment(nat, a, nat.size(), pp);
+    }
+    L.first[np] = (int)nat.size();
+    HIPCHK(ctx, dalloc(&L.d, all.size()));
+    HIPCHK(ctx, dalloc(&L.d_pp, pp.size()));
+    if (!all.empty()) HIPCHK(ctx, hipMemcpy(L.d, all.data(), all.size() * sizeof(TileCell), hipMemcpyHostToDevice));
+    if (!pp.empty()) HIPCHK(ctx, hipMemcpy(L.d_pp, pp.data(), pp.size() * sizeof(TileCell), hipMemcpyHostToDevice));
+  }
   return DRN_OK;
 }
 
@@ -925,6 +1034,10 @@ void drn_ctx_destroy(drn_ctx* ctx) {
     dfree(L.d_chain);
     L.d = L.d_xcd = L.d_xcd_pp = L.d_chain = nullptr;
   }
+  for (int w = 0; w < 2; ++w) {
+    free_box(ctx->box[w]);
+    free_box(ctx->box_rk[w]);
+  }
   dfree(ctx->d_mt_pp);
   dfree(ctx->d_mt_launch);
   dfree(ctx->d_thin_tiles);
@@ -1041,6 +1154,7 @@ int drn_layout(drn_ctx* ctx) {
       P.seek[f] = d.seek[f];
       for (int q = 0; q < 16; ++q) P.par[f][q] = d.bc_par[f][q];
     }
+    set_box(P, CellBox{0, d.ni, 0, d.nj, 0, d.nk});
     ctx->offs[p] = off;
     const uint64_t n = (uint64_t)d.ni * d.nj * d.nk;
     off += (n + ALIGN_CELLS - 1) / ALIGN_CELLS * ALIGN_CELLS;
@@ -1176,7 +1290,11 @@ int drn_layout(drn_ctx* ctx) {
   }
   HIPCHK(ctx, dalloc(&ctx->d_part, ctx->tiles.size() * 5));
   HIPCHK(ctx, dalloc(&ctx->d_out, 8));
-  int rc = build_march(ctx);
+  std::vector<std::vector<int>> one(np);
+  for (int p = 0; p < np; ++p) one[p].push_back(p);
+  int rc = build_box(ctx, pd, one, ctx->box);
+  if (rc) return rc;
+  rc = build_march(ctx);
   if (rc) return rc;
   ctx->laid_out = true;
   return DRN_OK;
@@ -1374,15 +1492,8 @@ static int patch_of(const drn_ctx* ctx, uint64_t g) {
 // together (plane i of every patch of the chain, then plane i + 1), so that
 // a donor's pushed rows and the receiver's own rows of the same lines are
 // written close together, by one XCD; then segmented per XCD as the others.
-static int build_chain_list(drn_ctx* ctx, const std::vector<std::pair<int, int>>& pairs) {
-  dfree(ctx->d_tz_chain);
-  ctx->d_tz_chain = nullptr;
-  for (auto& L : ctx->xs) {
-    dfree(L.d_chain);
-    L.d_chain = nullptr;
-  }
+static std::vector<std::vector<int>> push_chains(const drn_ctx* ctx, const std::vector<std::pair<int, int>>& pairs) {
   const int np = (int)ctx->descs.size();
-  if (pairs.empty() || np == 0) return DRN_OK;
   std::vector<int> up(np);
   for (int p = 0; p < np; ++p) up[p] = p;
   auto root = [&](int p) {
@@ -1403,6 +1514,17 @@ static int build_chain_list(drn_ctx* ctx, const std::vector<std::pair<int, int>>
     }
     chains[chain_of[r]].push_back(p);
   }
+  return chains;
+}
+
+static int build_chain_list(drn_ctx* ctx, const std::vector<std::vector<int>>& chains, bool linked) {
+  dfree(ctx->d_tz_chain);
+  ctx->d_tz_chain = nullptr;
+  for (auto& L : ctx->xs) {
+    dfree(L.d_chain);
+    L.d_chain = nullptr;
+  }
+  if (!linked) return DRN_OK;
   // items of xp planes x `cells` cells, the planes of a chain's patches side by
   // side, then in XCD segments
   auto chain_list = [&](int xp, int cells, size_t n_expect, TileCell** dptr) -> int {
@@ -1443,8 +1565,12 @@ int drn_exchange_commit(drn_ctx* ctx) {
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   drop_graph(ctx);  // a captured step holds the old lists
   free_exchange(ctx);
+  // without receivers no face is dead and every box is the whole patch
+  dfree(ctx->d_pd_rk);
+  ctx->d_pd_rk = nullptr;
+  for (auto& L : ctx->box_rk) free_box(L);
   for (PatchDev& P : ctx->pd_host) {
-    P.npush = P.nrecv = 0;
+    P.npush = P.nrecv = P.nrecv_box = 0;
     memset(P.push, 0, sizeof(P.push));
     memset(P.recv, 0, sizeof(P.recv));
   }
@@ -1532,6 +1658,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
       Q.push_si[sl] = (uint32_t)njk;
       Q.push_sj[sl] = (uint32_t)d.nk;
       P.recv[P.nrecv++] = CellBox{i0, i1, j0, j1, k0, k1};
+      P.nrecv_box = P.nrecv;
       push_pairs.push_back({q, p});
       for (int i = i0; i < i1; ++i)
         for (int j = j0; j < j1; ++j)
@@ -1677,6 +1804,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
   ctx->have_exchange = !ctx->xfull.single.empty() || ctx->xfull.multi_n > 0;
   ctx->n_fused = n_fused;
   HIPCHK(ctx, hipMemcpy(ctx->d_pd, ctx->pd_host.data(), ctx->pd_host.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
+  const std::vector<std::vector<int>> chains = push_chains(ctx, push_pairs);
   // Dead faces: a face with seek layers whose every boundary cell (the layer the
   // face functor acts on, cartesianiterator.h:190-308) is a receiver of the
   // exchange.  In the RK step the exchange after the stage overwrites those
@@ -1684,6 +1812,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
   {
     std::vector<PatchDev> rk = ctx->pd_host;
     int dead = 0;
+    bool trimmed = false;
     for (const auto& kv : ctx->xt) {
       const int p = kv.first;
       const drn_patch_desc& d = ctx->descs[p];
@@ -1709,16 +1838,43 @@ int drn_exchange_commit(drn_ctx* ctx) {
           ++dead;
         }
       }
+      // The box of the cells that are no receivers, the only ones whose new
+      // state survives that exchange: planes, rows and z layers of receivers
+      // around it are left out of the RK step's box lists.
+      CellBox b{d.ni, 0, d.nj, 0, d.nk, 0};
+      size_t l = 0;
+      for (int i = 0; i < d.ni; ++i)
+        for (int j = 0; j < d.nj; ++j)
+          for (int k = 0; k < d.nk; ++k, ++l) {
+            if (is_rec[l]) continue;
+            b.i0 = std::min(b.i0, i);
+            b.i1 = std::max(b.i1, i + 1);
+            b.j0 = std::min(b.j0, j);
+            b.j1 = std::max(b.j1, j + 1);
+            b.k0 = std::min(b.k0, k);
+            b.k1 = std::max(b.k1, k + 1);
+          }
+      if (b.i1 == 0) b = CellBox{0, 0, 0, 0, 0, 0};
+      trimmed = trimmed || b.i0 > 0 || b.i1 < d.ni || b.j0 > 0 || b.j1 < d.nj || b.k0 > 0 || b.k1 < d.nk;
+      PatchDev& P = rk[p];
+      set_box(P, b);
+      // the receive boxes that meet it come first
+      auto meets = [&](const CellBox& r) {
+        return std::max(r.i0, b.i0) < std::min(r.i1, b.i1) && std::max(r.j0, b.j0) < std::min(r.j1, b.j1) &&
+               std::max(r.k0, b.k0) < std::min(r.k1, b.k1);
+      };
+      if (P.nrecv == 2 && !meets(P.recv[0])) std::swap(P.recv[0], P.recv[1]);
+      P.nrecv_box = 0;
+      while (P.nrecv_box < P.nrecv && meets(P.recv[P.nrecv_box])) ++P.nrecv_box;
     }
-    dfree(ctx->d_pd_rk);
-    ctx->d_pd_rk = nullptr;
     ctx->n_dead_faces = dead;
-    if (dead > 0) {
+    if (dead > 0 || trimmed) {
       HIPCHK(ctx, dalloc(&ctx->d_pd_rk, rk.size()));
       HIPCHK(ctx, hipMemcpy(ctx->d_pd_rk, rk.data(), rk.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
+      if ((rc = build_box(ctx, rk, chains, ctx->box_rk))) return rc;
     }
   }
-  return build_chain_list(ctx, push_pairs);
+  return build_chain_list(ctx, chains, !push_pairs.empty());
 }
 
 int drn_set_exchange_fusion(drn_ctx* ctx, int on) {
@@ -2101,7 +2257,7 @@ int drn_set_tiling(drn_ctx* ctx, int launch, int choice) {
 
 int drn_get_tiling(const drn_ctx* ctx, int launch) {
   if (!ctx) return DRN_E_ARG;
-  return launch == DRN_LAUNCH_BATCHED ? ctx->tiling : ctx->tiling_pp;
+  return tiling_of(ctx, launch);
 }
 
 int drn_num_tilings(void) { return kNumTilings; }

@@ -324,7 +324,12 @@ int drn_post_variables(drn_ctx* ctx, int field, int patch, int mask, double ref_
  *       evaluations per cell; on the list of 35 (push chains) / XCD segmented;
  * 49, 50 the same over 2 planes per work item (two wavefronts per plane), 4.52
  *       face evaluations per cell.
- * Default for both forms: 11; drn_autotune picks per device. */
+ * 51, 52 the box kernel: as 47 / 48 over 1 or 4 planes per work item, but in
+ *       drn_rk_step and drn_rk_graph_run each patch's list covers only the box of
+ *       its cells that are no exchange receivers (the exchange after the stage
+ *       writes those), and the z slopes of a row are formed once per cell.
+ * Until a choice is set or autotuned, a rule on the size of the grid picks 51 or
+ * 52; drn_get_tiling returns the choice in effect. */
 int drn_num_tilings(void);
 int drn_set_tiling(drn_ctx* ctx, int launch, int choice);
 int drn_get_tiling(const drn_ctx* ctx, int launch);
