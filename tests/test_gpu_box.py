@@ -12,6 +12,7 @@ import pytest
 
 from drnum_amd import configs, hip
 from test_gpu_fused_exchange import run as run_fused
+from test_gpu_fused_exchange import setup as setup_fused
 from test_gpu_parity import TOL, make, rel_linf
 from test_gpu_thin import SHAPES, thin
 
@@ -150,3 +151,31 @@ def test_boxes_change_no_bit(gpu, dtype, make_w):
         for p, (a, b) in enumerate(zip(ref, got)):
             assert np.isfinite(a).all()
             assert np.array_equal(a, b), (fuse, choice, launch, p)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("viscous", [False, True])
+@pytest.mark.parametrize("launch", [B, PP])
+def test_boxes_of_the_flagged_and_the_viscous_operator(gpu, dtype, viscous, launch):
+    """The z-shared cell kernel, which these operators run, on the boxes' planes
+    and rows: every stored cell as with whole patches (boxes off), for row
+    lengths that end an item inside and beyond the box."""
+    for core in (5, 13, 18):
+        w = configs.viscous_shear(core=core, blocks=(2, 1, 2))
+        outs = []
+        for fuse in (False, True):
+            hg, ctx = setup_fused(w, dtype, fuse)
+            ctx.set_operator(w.recon, w.limiter, viscous)
+            if not viscous:
+                for p, P in enumerate(w.patches):
+                    flags = np.zeros(P.cells, np.uint8)
+                    flags[::7] = 1
+                    flags[3::11] |= 2
+                    ctx.set_cell_flags(p, flags)
+            for _ in range(3):
+                ctx.rk_step(w.dt, w.alpha, launch)
+            outs.append([ctx.download(p, 0) for p in range(len(w.patches))])
+            ctx.close()
+        for a, b in zip(*outs):
+            assert np.isfinite(a).all()
+            assert np.array_equal(a, b), core
