@@ -3151,59 +3151,79 @@ __device__ __forceinline__ double wave_min(double x) {
   return x;
 }
 
-// per-block partial sums of the core cells of one plane chunk (256 threads)
-template <typename T>
-__global__ __launch_bounds__(256) void k_sums_partial(const PatchDev* __restrict__ pds, const TileCell* __restrict__ tiles,
-                                                      const T* __restrict__ U, uint64_t vs, double* __restrict__ part) {
-  __shared__ double red[4][5];
-  const TileCell t = tiles[blockIdx.x];
-  const PatchDev& P = pds[t.patch];
-  const int c2 = t.c2 + (int)threadIdx.x;
-  double s[5] = {0, 0, 0, 0, 0};
-  if (c2 < P.njk) {
-    const int j = c2 / P.nk, k = c2 - j * P.nk, i = t.i;
-    const bool core = i >= P.seek[0] && i < P.ni - P.seek[1] && j >= P.seek[2] && j < P.nj - P.seek[3] &&
-                      k >= P.seek[4] && k < P.nk - P.seek[5];
-    if (core) {
-      const uint64_t c = (uint64_t)P.off + (uint64_t)i * P.njk + c2;
-      const double dV = P.dx * P.dy * P.dz;
-#pragma unroll
-      for (int v = 0; v < 5; ++v) s[v] = double(U[v * vs + c]) * dV;
-    }
-  }
+// The reductions run a grid that fills the device (kRedBlocksPerCu workgroups
+// per CU), each workgroup striding over the plane chunks, and one more workgroup
+// that combines the partials in a fixed order and leaves the result where the
+// caller reads it.  Both counts depend on the device and the grid only, so a
+// result is the same from call to call.  One partial per chunk instead, copied
+// to the host and combined there, took 283 us for the diagnostics of 8.5 M FP32
+// cells (170 MB, 30 us at the copy rate).
+enum { RED_SUM, RED_MAX, RED_MIN };
+template <int OP>
+__device__ __forceinline__ double red2(double a, double b) {
+  return OP == RED_SUM ? a + b : (OP == RED_MAX ? fmax(a, b) : fmin(a, b));
+}
+template <int OP>
+__device__ __forceinline__ double wave_red(double x) {
+  return OP == RED_SUM ? wave_sum(x) : (OP == RED_MAX ? wave_max(x) : wave_min(x));
+}
+
+// the workgroup's x[q] combined by OPS[q] (256 threads), into out[q]
+template <int... OPS>
+__device__ __forceinline__ void block_red(double* x, double* out) {
+  constexpr int N = sizeof...(OPS);
+  __shared__ double red[4][N];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int v = 0; v < 5; ++v) {
-    double x = wave_sum(s[v]);
-    if (lane == 0) red[wv][v] = x;
-  }
+  int q = 0;
+  (([&] {
+     const double y = wave_red<OPS>(x[q]);
+     if (lane == 0) red[wv][q] = y;
+     ++q;
+   }()),
+   ...);
   __syncthreads();
-  if (threadIdx.x < 5) {
-    const int v = threadIdx.x;
-    part[(uint64_t)blockIdx.x * 5 + v] = ((red[0][v] + red[1][v]) + red[2][v]) + red[3][v];
+  if (threadIdx.x == 0) {
+    q = 0;
+    ((out[q] = red2<OPS>(red2<OPS>(red2<OPS>(red[0][q], red[1][q]), red[2][q]), red[3][q]), ++q), ...);
   }
 }
 
-// fixed-order final sum of the partials (one block of 256)
-__global__ __launch_bounds__(256) void k_sums_final(uint32_t nblk, const double* __restrict__ part,
+// the partials of nblk workgroups combined (one workgroup)
+template <int... OPS>
+__global__ __launch_bounds__(256) void k_red_final(uint32_t nblk, const double* __restrict__ part,
                                                    double* __restrict__ out) {
-  __shared__ double red[4][5];
-  double s[5] = {0, 0, 0, 0, 0};
+  constexpr int N = sizeof...(OPS);
+  double x[N];
+  {
+    int q = 0;
+    ((x[q++] = OPS == RED_SUM ? 0.0 : (OPS == RED_MAX ? -1e300 : 1e300)), ...);
+  }
   for (uint32_t b = threadIdx.x; b < nblk; b += 256) {
+    int q = 0;
+    ((x[q] = red2<OPS>(x[q], part[(uint64_t)b * N + q]), ++q), ...);
+  }
+  block_red<OPS...>(x, out);
+}
+
+// FP64 sums of the conserved variables times dV over the core cells
+template <typename T>
+__global__ __launch_bounds__(256) void k_sums_partial(const PatchDev* __restrict__ pds, const TileCell* __restrict__ tiles,
+                                                      uint32_t nt, const T* __restrict__ U, uint64_t vs,
+                                                      double* __restrict__ part) {
+  double s[5] = {0, 0, 0, 0, 0};
+  for (uint32_t b = blockIdx.x; b < nt; b += gridDim.x) {
+    const TileCell t = tiles[b];
+    const PatchDev& P = pds[t.patch];
+    const int c2 = t.c2 + (int)threadIdx.x, i = t.i;
+    if (i < P.seek[0] || i >= P.ni - P.seek[1] || c2 >= P.njk) continue;
+    const int j = c2 / P.nk, k = c2 - j * P.nk;
+    if (j < P.seek[2] || j >= P.nj - P.seek[3] || k < P.seek[4] || k >= P.nk - P.seek[5]) continue;
+    const uint64_t c = (uint64_t)P.off + (uint64_t)i * P.njk + c2;
+    const double dV = P.dx * P.dy * P.dz;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) s[v] += part[(uint64_t)b * 5 + v];
+    for (int v = 0; v < 5; ++v) s[v] += double(U[v * vs + c]) * dV;
   }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int v = 0; v < 5; ++v) {
-    double x = wave_sum(s[v]);
-    if (lane == 0) red[wv][v] = x;
-  }
-  __syncthreads();
-  if (threadIdx.x < 5) {
-    const int v = threadIdx.x;
-    out[v] = ((red[0][v] + red[1][v]) + red[2][v]) + red[3][v];
-  }
+  block_red<RED_SUM, RED_SUM, RED_SUM, RED_SUM, RED_SUM>(s, part + 5 * (uint64_t)blockIdx.x);
 }
 
 // The CFL number of one cell as the jet demo computes it
@@ -3211,117 +3231,81 @@ __global__ __launch_bounds__(256) void k_sums_final(uint32_t nblk, const double*
 // (perfectgas.h:84-92) and a = sqrt(gamma R T) in the state type, with the
 // reference's double-literal promotions (1.0/rho, 0.5*|u|^2, /cv), then
 // max(|u|, |u+a|, |u-a|) * dt / dx with the x velocity and spacing only.
+// ird = 1.0 / rho in double.  The three products and quotients are monotone in
+// their first factor, so the largest of the three numbers is that of the largest.
 template <typename T>
-__device__ __forceinline__ T cfl_x_reference(const T* var, T dt, T dx) {
+__device__ __forceinline__ T cfl_x_reference(const T* var, double ird, T dt, T dx) {
 #pragma clang fp contract(off)
-  const T ir = T(1.0 / double(var[0]));
+  const T ir = T(ird);
   const T u = var[1] * ir, v = var[2] * ir, w = var[3] * ir;
   const T Tt = T((double(var[4] * ir) - 0.5 * double(u * u + v * v + w * w)) / double(Gas<T>::CV));
   const T a = dsqrt(Gas<T>::GAMMA * Gas<T>::R * Tt);
-  T c = dabs(u) * dt / dx;
-  c = fmax(c, dabs(u + a) * dt / dx);
-  c = fmax(c, dabs(u - a) * dt / dx);
-  return c;
+  return fmax(dabs(u), fmax(dabs(u + a), dabs(u - a))) * dt / dx;
 }
 
-// diagnostics partials per tile: [0] the reference CFL (x axis only), [1] min
-// rho, [2] max rho, [3] count of non-finite values, [4] the CFL over all three
+// diagnostics: [0] the reference CFL (x axis only; AXES: 0), [1] min rho, [2]
+// max rho, [3] count of non-finite values, [4] AXES: the CFL over all three
 // axes, max_d (|u_d| + a) dt / d_d, evaluated in FP64
-template <typename T>
+template <typename T, bool AXES>
 __global__ __launch_bounds__(256) void k_diag_partial(const PatchDev* __restrict__ pds, const TileCell* __restrict__ tiles,
-                                                      const T* __restrict__ U, uint64_t vs, double dt,
+                                                      uint32_t nt, const T* __restrict__ U, uint64_t vs, double dt,
                                                       double* __restrict__ part) {
-  __shared__ double red[4][5];
-  const TileCell t = tiles[blockIdx.x];
-  const PatchDev& P = pds[t.patch];
-  const int c2 = t.c2 + (int)threadIdx.x;
   double cflx = 0, cfl3 = 0, rmin = 1e300, rmax = -1e300, bad = 0;
-  if (c2 < P.njk) {
+  for (uint32_t b = blockIdx.x; b < nt; b += gridDim.x) {
+    const TileCell t = tiles[b];
+    const PatchDev& P = pds[t.patch];
+    const int c2 = t.c2 + (int)threadIdx.x;
+    if (c2 >= P.njk) continue;
     const uint64_t c = (uint64_t)P.off + (uint64_t)t.i * P.njk + c2;
     T tv[5];
     double var[5];
 #pragma unroll
+    for (int v = 0; v < 5; ++v) tv[v] = U[v * vs + c];
+#pragma unroll
     for (int v = 0; v < 5; ++v) {
-      tv[v] = U[v * vs + c];
       var[v] = double(tv[v]);
       if (!isfinite(var[v])) bad += 1;
     }
-    cflx = double(cfl_x_reference<T>(tv, T(dt), T(P.dx)));
-    if (!isfinite(cflx)) cflx = 0;
-    double ir = 1.0 / var[0];
-    double u = var[1] * ir, v = var[2] * ir, w = var[3] * ir;
-    double Tt = (var[4] * ir - 0.5 * (u * u + v * v + w * w)) / 717.5;
-    double a = sqrt(1.4 * 287.2 * Tt);
-    cfl3 = fmax(fmax((fabs(u) + a) * dt / P.dx, (fabs(v) + a) * dt / P.dy), (fabs(w) + a) * dt / P.dz);
-    if (!isfinite(cfl3)) cfl3 = 0;
-    rmin = var[0];
-    rmax = var[0];
-  }
-  cflx = wave_max(cflx);
-  cfl3 = wave_max(cfl3);
-  rmin = wave_min(rmin);
-  rmax = wave_max(rmax);
-  bad = wave_sum(bad);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    red[wv][0] = cflx;
-    red[wv][1] = rmin;
-    red[wv][2] = rmax;
-    red[wv][3] = bad;
-    red[wv][4] = cfl3;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double o[5] = {red[0][0], red[0][1], red[0][2], red[0][3], red[0][4]};
-    for (int q = 1; q < 4; ++q) {
-      o[0] = fmax(o[0], red[q][0]);
-      o[1] = fmin(o[1], red[q][1]);
-      o[2] = fmax(o[2], red[q][2]);
-      o[3] += red[q][3];
-      o[4] = fmax(o[4], red[q][4]);
+    const double ir = 1.0 / var[0];
+    if constexpr (AXES) {
+      const double u = var[1] * ir, v = var[2] * ir, w = var[3] * ir;
+      const double Tt = (var[4] * ir - 0.5 * (u * u + v * v + w * w)) / 717.5;
+      const double a = sqrt(1.4 * 287.2 * Tt);
+      const double x = fmax(fmax((fabs(u) + a) * dt / P.dx, (fabs(v) + a) * dt / P.dy), (fabs(w) + a) * dt / P.dz);
+      if (isfinite(x)) cfl3 = fmax(cfl3, x);
+    } else {
+      const double x = double(cfl_x_reference<T>(tv, ir, T(dt), T(P.dx)));
+      if (isfinite(x)) cflx = fmax(cflx, x);
     }
-#pragma unroll
-    for (int q = 0; q < 5; ++q) part[(uint64_t)blockIdx.x * 5 + q] = o[q];
+    rmin = fmin(rmin, var[0]);
+    rmax = fmax(rmax, var[0]);
   }
+  double x[5] = {cflx, rmin, rmax, bad, cfl3};
+  block_red<RED_MAX, RED_MIN, RED_MAX, RED_SUM, RED_MAX>(x, part + 5 * (uint64_t)blockIdx.x);
 }
 
 // Patch::computeVariableDifference (patch.cpp:733-746) over the cells of one
-// patch's tiles: per cell (b - a)^2 in the state type; per block its maximum
-// (exactly a state-type value) and its FP64 sum.
+// patch's tiles: per cell (b - a)^2 in the state type; its maximum (exactly a
+// state-type value) and its FP64 sum.
 template <typename T>
 __global__ __launch_bounds__(256) void k_vardiff_partial(const PatchDev* __restrict__ pds,
-                                                         const TileCell* __restrict__ tiles, const T* __restrict__ a,
-                                                         const T* __restrict__ b, double* __restrict__ part) {
+                                                         const TileCell* __restrict__ tiles, uint32_t nt,
+                                                         const T* __restrict__ a, const T* __restrict__ b,
+                                                         double* __restrict__ part) {
 #pragma clang fp contract(off)
-  __shared__ double red[4][2];
-  const TileCell t = tiles[blockIdx.x];
-  const PatchDev& P = pds[t.patch];
-  const int c2 = t.c2 + (int)threadIdx.x;
-  double mx = 0, sum = 0;
-  if (c2 < P.njk) {
+  double x[2] = {0, 0};
+  for (uint32_t q = blockIdx.x; q < nt; q += gridDim.x) {
+    const TileCell t = tiles[q];
+    const PatchDev& P = pds[t.patch];
+    const int c2 = t.c2 + (int)threadIdx.x;
+    if (c2 >= P.njk) continue;
     const uint64_t c = (uint64_t)P.off + (uint64_t)t.i * P.njk + c2;
     const T d = b[c] - a[c];
     const T sq = d * d;
-    mx = double(sq);
-    sum = double(sq);
+    x[0] = fmax(x[0], double(sq));
+    x[1] += double(sq);
   }
-  mx = wave_max(mx);
-  sum = wave_sum(sum);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    red[wv][0] = mx;
-    red[wv][1] = sum;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double o0 = red[0][0], o1 = red[0][1];
-    for (int q = 1; q < 4; ++q) {
-      o0 = fmax(o0, red[q][0]);
-      o1 += red[q][1];
-    }
-    part[(uint64_t)blockIdx.x * 2 + 0] = o0;
-    part[(uint64_t)blockIdx.x * 2 + 1] = o1;
-  }
+  block_red<RED_MAX, RED_SUM>(x, part + 2 * (uint64_t)blockIdx.x);
 }
 
 }  // namespace drn

@@ -20,6 +20,7 @@ namespace {
 
 constexpr int NBUF = 3;
 constexpr int ALIGN_CELLS = 64;
+constexpr int kRedBlocksPerCu = 8;  // a full device of 256-thread workgroups
 
 struct ExchangeTables {
   // reference form, per receiver patch (local cell indices)
@@ -120,8 +121,9 @@ struct drn_ctx {
   TileCell* d_tyz = nullptr;
   TileCell* d_tyz_xcd = nullptr;
   TileCell* d_tyz_xcd_pp = nullptr;
-  double* d_part = nullptr;  // reduction partials (5 per tile)
-  double* d_out = nullptr;
+  double* d_part = nullptr;  // reduction partials (5 per workgroup)
+  double* h_out = nullptr;   // pinned: results of the reductions
+  double* d_hout = nullptr;  // its device address
   void* d_post = nullptr;    // post-processing output of one patch
   size_t post_bytes = 0;
   int tiling = -1;     // batched form; -1: by auto_tiling until one is set
@@ -1057,7 +1059,7 @@ void drn_ctx_destroy(drn_ctx* ctx) {
   dfree(ctx->d_wt_pp);
   dfree(ctx->d_wt_launch);
   dfree(ctx->d_part);
-  dfree(ctx->d_out);
+  if (ctx->h_out) (void)hipHostFree(ctx->h_out);
   dfree(ctx->d_post);
   for (auto& s : ctx->timers) {
     for (auto& e : s.used) {
@@ -1301,8 +1303,9 @@ int drn_layout(drn_ctx* ctx) {
     HIPCHK(ctx, hipMemcpy(ctx->d_tx2_xcd, xall.data(), n2 * sizeof(TileCell), hipMemcpyHostToDevice));
     HIPCHK(ctx, hipMemcpy(ctx->d_tx2_xcd_pp, xpp.data(), n2 * sizeof(TileCell), hipMemcpyHostToDevice));
   }
-  HIPCHK(ctx, dalloc(&ctx->d_part, ctx->tiles.size() * 5));
-  HIPCHK(ctx, dalloc(&ctx->d_out, 8));
+  HIPCHK(ctx, dalloc(&ctx->d_part, (size_t)kRedBlocksPerCu * ctx->n_cu * 5));
+  HIPCHK(ctx, hipHostMalloc((void**)&ctx->h_out, 8 * sizeof(double), hipHostMallocDefault));
+  HIPCHK(ctx, hipHostGetDevicePointer((void**)&ctx->d_hout, ctx->h_out, 0));
   std::vector<std::vector<int>> one(np);
   for (int p = 0; p < np; ++p) one[p].push_back(p);
   int rc = build_box(ctx, pd, one, ctx->box, 2);
@@ -2072,15 +2075,24 @@ int drn_rk_graph_run(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, 
   return DRN_OK;
 }
 
+// workgroups of a reduction over nt plane chunks
+static int red_blocks(const drn_ctx* ctx, int nt) { return std::max(1, std::min(nt, kRedBlocksPerCu * ctx->n_cu)); }
+
+// the sums' two kernels, the partials in `part`
 template <typename T>
-static int sums_t(drn_ctx* ctx, const T* U, double* out) {
-  const int nt = (int)ctx->tiles.size();
-  hipLaunchKernelGGL(k_sums_partial<T>, dim3(nt), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles, U, ctx->vstride,
-                     ctx->d_part);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(256), 0, ctx->stream, (uint32_t)nt, ctx->d_part, ctx->d_out);
+static void launch_sums(drn_ctx* ctx, const T* U, double* part, double* out) {
+  const int nt = (int)ctx->tiles.size(), nb = red_blocks(ctx, nt);
+  hipLaunchKernelGGL(k_sums_partial<T>, dim3(nb), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles, (uint32_t)nt, U,
+                     ctx->vstride, part);
+  hipLaunchKernelGGL((k_red_final<RED_SUM, RED_SUM, RED_SUM, RED_SUM, RED_SUM>), dim3(1), dim3(256), 0, ctx->stream,
+                     (uint32_t)nb, part, out);
+}
+
+// the first n doubles of h_out, once the stream has written them
+static int read_out(drn_ctx* ctx, double* out, int n) {
   HIPCHK(ctx, hipGetLastError());
-  HIPCHK(ctx, hipMemcpyAsync(out, ctx->d_out, 5 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  memcpy(out, ctx->h_out, n * sizeof(double));
   return DRN_OK;
 }
 
@@ -2090,21 +2102,17 @@ int drn_core_sums(drn_ctx* ctx, int field, double* out) {
   if ((rc = check_field(ctx, field))) return rc;
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const void* U = ctx->buf[ctx->map[field]];
-  return ctx->prec == DRN_F32 ? sums_t(ctx, (const float*)U, out) : sums_t(ctx, (const double*)U, out);
+  if (ctx->prec == DRN_F32)
+    launch_sums(ctx, (const float*)U, ctx->d_part, ctx->d_hout);
+  else
+    launch_sums(ctx, (const double*)U, ctx->d_part, ctx->d_hout);
+  return read_out(ctx, out, 5);
 }
 
 // drn_core_sums with the partials in `scratch` (through its device address
 // ctx->scratch) and the result left in device memory: the same kernels, so the
-// same sums bit for bit.  Every partial row read by k_sums_final is written by
+// same sums bit for bit.  Every partial row read by k_red_final is written by
 // k_sums_partial of the same call, so nothing needs clearing.
-template <typename T>
-static void sums_noalloc_t(drn_ctx* ctx, const T* U, double* d_out) {
-  const int nt = (int)ctx->tiles.size();
-  hipLaunchKernelGGL(k_sums_partial<T>, dim3(nt), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles, U, ctx->vstride,
-                     ctx->scratch);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(256), 0, ctx->stream, (uint32_t)nt, ctx->scratch, d_out);
-}
-
 int drn_core_sums_noalloc(drn_ctx* ctx, int field, double* d_out) {
   if (!ctx || !d_out) return DRN_E_ARG;
   int rc;
@@ -2118,48 +2126,40 @@ int drn_core_sums_noalloc(drn_ctx* ctx, int field, double* d_out) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const void* U = ctx->buf[ctx->map[field]];
   if (ctx->prec == DRN_F32)
-    sums_noalloc_t(ctx, (const float*)U, d_out);
+    launch_sums(ctx, (const float*)U, ctx->scratch, d_out);
   else
-    sums_noalloc_t(ctx, (const double*)U, d_out);
+    launch_sums(ctx, (const double*)U, ctx->scratch, d_out);
   HIPCHK(ctx, hipGetLastError());
   return DRN_OK;
 }
 
-// out[0..4] as k_diag_partial's partials, reduced over all tiles
+// out[0..4] as k_diag_partial describes them
 template <typename T>
-static int diag_t(drn_ctx* ctx, const T* U, double dt, double* out) {
-  const int nt = (int)ctx->tiles.size();
-  hipLaunchKernelGGL(k_diag_partial<T>, dim3(nt), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles, U, ctx->vstride,
+static void launch_diag(drn_ctx* ctx, const T* U, double dt, bool axes) {
+  const int nt = (int)ctx->tiles.size(), nb = red_blocks(ctx, nt);
+  const auto kern = axes ? k_diag_partial<T, true> : k_diag_partial<T, false>;
+  hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles, (uint32_t)nt, U, ctx->vstride,
                      dt, ctx->d_part);
-  HIPCHK(ctx, hipGetLastError());
-  std::vector<double> h((size_t)nt * 5);
-  HIPCHK(ctx, hipMemcpyAsync(h.data(), ctx->d_part, h.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  double o[5] = {0, 1e300, -1e300, 0, 0};
-  for (int b = 0; b < nt; ++b) {
-    o[0] = std::max(o[0], h[5 * b]);
-    o[1] = std::min(o[1], h[5 * b + 1]);
-    o[2] = std::max(o[2], h[5 * b + 2]);
-    o[3] += h[5 * b + 3];
-    o[4] = std::max(o[4], h[5 * b + 4]);
-  }
-  memcpy(out, o, sizeof(o));
-  return DRN_OK;
+  hipLaunchKernelGGL((k_red_final<RED_MAX, RED_MIN, RED_MAX, RED_SUM, RED_MAX>), dim3(1), dim3(256), 0, ctx->stream,
+                     (uint32_t)nb, ctx->d_part, ctx->d_hout);
 }
 
-static int diag(drn_ctx* ctx, int field, double dt, double* o5) {
+static int diag(drn_ctx* ctx, int field, double dt, bool axes, double* o5) {
   int rc;
   if ((rc = check_field(ctx, field))) return rc;
-  if (!ctx->laid_out) return fail(ctx, DRN_E_STATE, "drn_layout not called");
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const void* U = ctx->buf[ctx->map[field]];
-  return ctx->prec == DRN_F32 ? diag_t(ctx, (const float*)U, dt, o5) : diag_t(ctx, (const double*)U, dt, o5);
+  if (ctx->prec == DRN_F32)
+    launch_diag(ctx, (const float*)U, dt, axes);
+  else
+    launch_diag(ctx, (const double*)U, dt, axes);
+  return read_out(ctx, o5, 5);
 }
 
 int drn_diagnostics(drn_ctx* ctx, int field, double dt, double* out) {
   if (!ctx || !out) return DRN_E_ARG;
   double o[5];
-  int rc = diag(ctx, field, dt, o);
+  int rc = diag(ctx, field, dt, false, o);
   if (rc) return rc;
   memcpy(out, o, 4 * sizeof(double));
   return DRN_OK;
@@ -2168,7 +2168,7 @@ int drn_diagnostics(drn_ctx* ctx, int field, double dt, double* out) {
 int drn_cfl_axes(drn_ctx* ctx, int field, double dt, double* cfl) {
   if (!ctx || !cfl) return DRN_E_ARG;
   double o[5];
-  int rc = diag(ctx, field, dt, o);
+  int rc = diag(ctx, field, dt, true, o);
   if (rc) return rc;
   *cfl = o[4];
   return DRN_OK;
@@ -2176,20 +2176,14 @@ int drn_cfl_axes(drn_ctx* ctx, int field, double dt, double* cfl) {
 
 template <typename T>
 static int vardiff_t(drn_ctx* ctx, int patch, const T* a, const T* b, double* max_norm, double* l2_norm) {
-  const int t0 = ctx->tile_first[patch], nt = ctx->tile_first[patch + 1] - t0;
-  if (nt > 0)
-    hipLaunchKernelGGL(k_vardiff_partial<T>, dim3(nt), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles + t0, a, b,
-                       ctx->d_part);
-  HIPCHK(ctx, hipGetLastError());
-  std::vector<double> h((size_t)nt * 2);
-  if (nt > 0)
-    HIPCHK(ctx, hipMemcpyAsync(h.data(), ctx->d_part, h.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  double mx = 0, sum = 0;
-  for (int q = 0; q < nt; ++q) {
-    mx = std::max(mx, h[2 * q]);
-    sum += h[2 * q + 1];
-  }
+  const int t0 = ctx->tile_first[patch], nt = ctx->tile_first[patch + 1] - t0, nb = red_blocks(ctx, nt);
+  hipLaunchKernelGGL(k_vardiff_partial<T>, dim3(nb), dim3(256), 0, ctx->stream, ctx->d_pd, ctx->d_tiles + t0,
+                     (uint32_t)nt, a, b, ctx->d_part);
+  hipLaunchKernelGGL((k_red_final<RED_MAX, RED_SUM>), dim3(1), dim3(256), 0, ctx->stream, (uint32_t)nb, ctx->d_part,
+                     ctx->d_hout);
+  double o[2];
+  if (const int rc = read_out(ctx, o, 2)) return rc;
+  const double mx = std::max(0.0, o[0]), sum = o[1];
   // the maximum is a state-type value: its square root in the state type, as
   // the reference takes it; the sum was accumulated in FP64
   *max_norm = (double)std::sqrt((T)mx);
