@@ -2905,6 +2905,30 @@ __global__ __launch_bounds__(256) void k_copy(uint64_t n16, const uint4* __restr
   for (uint64_t q = blockIdx.x * 256ull + threadIdx.x; q < n16; q += (uint64_t)gridDim.x * 256ull) dst[q] = src[q];
 }
 
+// Between one patch's 5 x n values in the host layout (variable after variable)
+// and the variable arrays: values [e0, e0 + cnt) of the patch, whose value e =
+// v n + l lives at arr[v * vs + l], to or from the pinned host memory `host`.
+// The kernel reads or writes it across the host link itself: one launch per
+// piece instead of one copy per variable.  V = uint4: 16 bytes per lane, for n,
+// e0 and cnt multiples of the values in it (vs and arr are multiples of 64 cells).
+template <typename V, typename E, bool TO_HOST>
+__global__ __launch_bounds__(256) void k_host_copy(E* arr, uint64_t vs, uint64_t n, uint64_t e0, uint32_t cnt, V* host) {
+  constexpr uint32_t M = sizeof(V) / sizeof(E);
+  const uint64_t v0 = e0 / n, l0 = e0 - v0 * n;
+  for (uint32_t q = blockIdx.x * 256u + threadIdx.x; q < cnt / M; q += gridDim.x * 256u) {
+    uint64_t l = l0 + (uint64_t)q * M, v = v0;
+    while (l >= n) {
+      l -= n;
+      ++v;
+    }
+    V* d = reinterpret_cast<V*>(arr + v * vs + l);
+    if constexpr (TO_HOST)
+      host[q] = *d;
+    else
+      *d = host[q];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // exchange (gather): receivers are seek cells, donors are donor-zone cells of
 // other patches, so the two sets never intersect and all receivers of all
