@@ -248,6 +248,11 @@ struct drn_ctx {
     void* m_turn = nullptr;    // 9 values per turn matrix, in the state precision
   };
   ExchangeLists xfull, xpart;
+  // the receivers that a level-set fill can change the exchange of: filled
+  // cells, and receivers with a filled donor
+  ExchangeLists xls;
+  bool xls_ok = false;  // xls belongs to the committed tables of both kinds
+  bool xt_dirty = false, lt_dirty = false;  // tables set since their last commit
   bool have_exchange = false;
   std::vector<PatchDev> pd_host;  // the device patch descriptors as uploaded
   bool fuse = true;               // drn_set_exchange_fusion
@@ -273,7 +278,7 @@ struct drn_ctx {
     double dt;
     std::vector<double> alpha;
     int steps;      // steps per replay (the cycle of the field-map permutation)
-    int exch_end;   // exch_buf after one replay
+    int exch_end, exch_ls_end;  // exch_buf and exch_ls_buf after one replay
     hipGraphExec_t exec;
   };
   std::vector<GraphEntry> graphs;
@@ -282,6 +287,9 @@ struct drn_ctx {
   // buffer; a step without post operation skips its leading exchange
   // (rungekutta.cpp:30) only when it is set for the state buffer.
   int exch_buf = -1;
+  // The same but for the receivers of xls: a level-set fill changed cells of the
+  // buffer since its exchange, and nothing else did (-1: none).
+  int exch_ls_buf = -1;
 
   size_t esize() const { return prec == DRN_F32 ? 4 : 8; }
 };
@@ -303,6 +311,7 @@ static void drop_graph(drn_ctx* ctx) {
 // buffer b is written: its receivers no longer hold the exchange
 static void wrote(drn_ctx* ctx, int b) {
   if (ctx->exch_buf == b) ctx->exch_buf = -1;
+  if (ctx->exch_ls_buf == b) ctx->exch_ls_buf = -1;
 }
 
 static int fail(drn_ctx* ctx, int code, const std::string& msg) {
@@ -926,10 +935,12 @@ static void launch_exchange_t(drn_ctx* ctx, const drn_ctx::ExchangeLists& x, T* 
   }
 }
 
-// partial: the stage just launched filled the fused z-face receivers itself
-static int do_exchange(drn_ctx* ctx, int pbuf, bool partial = false) {
+// which receivers an exchange copies: all; all but the fused z-face receivers,
+// which the stage just launched filled itself; or those a level-set fill touched
+enum { X_FULL, X_PART, X_LS };
+static int do_exchange(drn_ctx* ctx, int pbuf, int which = X_FULL) {
   if (!ctx->have_exchange) return DRN_OK;
-  const drn_ctx::ExchangeLists& x = partial ? ctx->xpart : ctx->xfull;
+  const drn_ctx::ExchangeLists& x = which == X_PART ? ctx->xpart : (which == X_LS ? ctx->xls : ctx->xfull);
   hipEvent_t stop;
   timer_begin(ctx, 1, &stop);
   if (ctx->prec == DRN_F32)
@@ -938,8 +949,10 @@ static int do_exchange(drn_ctx* ctx, int pbuf, bool partial = false) {
     launch_exchange_t<double>(ctx, x, (double*)ctx->buf[pbuf]);
   timer_end(ctx, stop);
   HIPCHK(ctx, hipGetLastError());
-  // after a stage that filled the fused receivers, the partial lists complete the exchange
+  // after a stage that filled the fused receivers, the partial lists complete the
+  // exchange; after a fill that alone changed an exchanged buffer, xls does
   ctx->exch_buf = pbuf;
+  if (ctx->exch_ls_buf == pbuf) ctx->exch_ls_buf = -1;
   return DRN_OK;
 }
 
@@ -958,7 +971,9 @@ static void launch_ls_t(drn_ctx* ctx, T* U, T relax) {
 
 static int do_ls_fill(drn_ctx* ctx, int pbuf, double relax) {
   if (ctx->ls_n == 0) return DRN_OK;
+  const bool exchanged = ctx->exch_buf == pbuf || ctx->exch_ls_buf == pbuf;
   wrote(ctx, pbuf);
+  if (exchanged) ctx->exch_ls_buf = pbuf;
   hipEvent_t stop;
   timer_begin(ctx, 2, &stop);
   if (ctx->prec == DRN_F32)
@@ -982,19 +997,22 @@ static int do_rk_step(drn_ctx* ctx, double dt, int n_alpha, const double* alpha,
   int Z = 0;
   while (Z == X || Z == Y) ++Z;
   int rc;
-  if (post || ctx->exch_buf != X) {
-    if ((rc = do_exchange(ctx, X))) return rc;
-  }
+  // the exchange before a stage: nothing to do for a buffer that holds it, the
+  // receivers a fill touched where only a fill came after it
+  auto lead = [&](int b) {
+    return ctx->exch_buf == b ? (int)DRN_OK : do_exchange(ctx, b, ctx->exch_ls_buf == b && ctx->xls_ok ? X_LS : X_FULL);
+  };
+  if ((rc = lead(X))) return rc;
   int cur = X;
   // the stage fills the fused z-face receivers, the exchange after it the rest
   const bool push = push_active(ctx, launch);
   for (int s = 0; s < n_alpha; ++s) {
     if (s > 0 && post) {
-      if ((rc = do_exchange(ctx, cur))) return rc;
+      if ((rc = lead(cur))) return rc;
     }
     const int dst = (s % 2 == 0) ? Y : Z;
     if ((rc = do_stage(ctx, cur, X, dst, alpha[s] * dt, launch, push, true))) return rc;
-    if ((rc = do_exchange(ctx, dst, push))) return rc;
+    if ((rc = do_exchange(ctx, dst, push ? X_PART : X_FULL))) return rc;
     if (post) {
       if ((rc = do_ls_fill(ctx, dst, 0.5))) return rc;
     }
@@ -1086,6 +1104,9 @@ static void free_lists(drn_ctx::ExchangeLists& x) {
 static void free_exchange(drn_ctx* ctx) {
   free_lists(ctx->xfull);
   free_lists(ctx->xpart);
+  free_lists(ctx->xls);
+  ctx->xls_ok = false;
+  ctx->exch_buf = ctx->exch_ls_buf = -1;
   ctx->have_exchange = false;
   ctx->n_fused = 0;
 }
@@ -1614,6 +1635,7 @@ int drn_exchange_set(drn_ctx* ctx, int recv_id, int n_donors, const int32_t* don
   for (int64_t a = 0; a < n_unique; ++a)
     if (t.rec_unique[a] < 0 || t.rec_unique[a] >= nrecv_cells) return fail(ctx, DRN_E_RANGE, "receiver cell outside patch");
   ctx->xt[recv_id] = std::move(t);
+  ctx->xt_dirty = true;
   return DRN_OK;
 }
 
@@ -1627,6 +1649,7 @@ int drn_exchange_set_turn(drn_ctx* ctx, int recv_id, int n_donors, const double*
   for (int64_t a = 0; a < 9 * (int64_t)n_donors; ++a)
     if (!std::isfinite(turn[a])) return fail(ctx, DRN_E_ARG, "drn_exchange_set_turn: non-finite matrix entry");
   it->second.turn.assign(turn, turn + 9 * (size_t)n_donors);
+  ctx->xt_dirty = true;
   return DRN_OK;
 }
 
@@ -1727,6 +1750,20 @@ static int build_chain_list(drn_ctx* ctx, const std::vector<std::vector<int>>& c
   return chain_list(4, 63, ctx->xs[1].nat.size(), &ctx->xs[1].d_chain);
 }
 
+// one donor's contribution to one receiver: global donor cells and weights
+struct DonorGroup {
+  int stride;
+  int turn = 0;  // 0 = aligned, t > 0 = matrix t - 1 of the list's turn matrices
+  std::vector<uint32_t> idx;
+  std::vector<double> w;
+};
+typedef std::pair<uint32_t, std::vector<DonorGroup>> ExchangeReceiver;  // global cell, its groups in donor order
+
+static int upload_multi(drn_ctx* ctx, drn_ctx::ExchangeLists& x,
+                        std::vector<std::pair<size_t, const ExchangeReceiver*>>& order,
+                        const std::vector<double>& turns);
+static int build_ls_exchange(drn_ctx* ctx);
+
 int drn_exchange_commit(drn_ctx* ctx) {
   if (!ctx) return DRN_E_ARG;
   if (!ctx->laid_out) return fail(ctx, DRN_E_STATE, "drn_layout not called");
@@ -1743,13 +1780,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
     memset(P.push, 0, sizeof(P.push));
     memset(P.recv, 0, sizeof(P.recv));
   }
-  // per unique receiver: its contribution groups in donor order
-  struct Group {
-    int stride;
-    int turn = 0;  // 0 = aligned, t > 0 = matrix t - 1 of `turns`
-    std::vector<uint32_t> idx;
-    std::vector<double> w;
-  };
+  typedef DonorGroup Group;  // per unique receiver: its contribution groups in donor order
   std::vector<double> turns;  // 9 per turned (receiver patch, donor) relation
   std::map<int, std::vector<std::pair<uint32_t, std::vector<Group>>>> single_by_stride;
   std::vector<std::pair<uint32_t, std::vector<Group>>> multi;
@@ -1901,13 +1932,6 @@ int drn_exchange_commit(drn_ctx* ctx) {
       x.single.push_back(c);  // freed with the lists, also after a failed upload
       if (rc) return fail(ctx, DRN_E_NOMEM, "exchange list upload failed");
     }
-    // the multi-donor receivers, sorted by their number of entries in bands
-    // of 8 (descending), so that the 64 lanes of a wavefront loop over about
-    // as many entries each, and within a band by their first donor cell, so
-    // that the lanes read neighbouring donor cells: on a 200-patch nested
-    // batch 0.356 ms per exchange, against 0.564 sorted by the count alone,
-    // 0.387 with bands of 1 and 0.385 by the donor cell alone;
-    // wavefront b's entries start at tbase[b], entry q of lane L at + 64 q + L
     std::vector<std::pair<size_t, const std::pair<uint32_t, std::vector<Group>>*>> order;  // (entries, receiver)
     for (const auto& e : multi) {
       if (skip_fused && fused[e.first]) continue;
@@ -1922,55 +1946,12 @@ int drn_exchange_commit(drn_ctx* ctx) {
         order.push_back({e.second[0].idx.size(), &e});
       }
     }
-    auto first_donor = [](const std::pair<uint32_t, std::vector<Group>>* e) -> uint32_t {
-      return e->second.empty() || e->second[0].idx.empty() ? 0u : e->second[0].idx[0];
-    };
-    std::stable_sort(order.begin(), order.end(), [&](const auto& a, const auto& b) {
-      const size_t ka = (a.first + 7) / 8, kb = (b.first + 7) / 8;
-      if (ka != kb) return ka > kb;
-      return first_donor(a.second) < first_donor(b.second);
-    });
-    std::vector<uint32_t> rec, cnt, tbase, ent, et;
-    std::vector<double> w;
-    const bool turned = !turns.empty();
-    for (size_t b = 0; b < order.size(); b += 64) {
-      const size_t nb = std::min<size_t>(64, order.size() - b);
-      size_t emax = 0;
-      for (size_t L = 0; L < nb; ++L) emax = std::max(emax, order[b + L].first);
-      if (ent.size() + 64 * emax > 0xffffffffu) return fail(ctx, DRN_E_RANGE, "exchange lists exceed 2^32 entries");
-      tbase.push_back((uint32_t)ent.size());
-      ent.resize(ent.size() + 64 * emax, 0u);
-      w.resize(ent.size(), 0.0);
-      if (turned) et.resize(ent.size(), 0u);
-      for (size_t L = 0; L < nb; ++L) {
-        const auto& e = *order[b + L].second;
-        rec.push_back(e.first);
-        size_t q = 0;
-        for (const auto& g : e.second) {
-          for (size_t s2 = 0; s2 < g.idx.size(); ++s2, ++q) {
-            const size_t at = tbase.back() + 64 * q + L;
-            if (g.idx[s2] & 0x80000000u) return fail(ctx, DRN_E_RANGE, "donor cell index beyond 2^31");
-            ent[at] = g.idx[s2] | (s2 + 1 == g.idx.size() ? 0x80000000u : 0u);
-            w[at] = g.w[s2];
-            if (turned && s2 + 1 == g.idx.size()) et[at] = (uint32_t)g.turn;
-          }
-        }
-        cnt.push_back((uint32_t)q);
-      }
-    }
-    if (!rec.empty()) {
-      x.multi_n = (uint32_t)rec.size();
-      if (upload_vec(ctx, &x.m_rec, rec) || upload_vec(ctx, &x.m_cnt, cnt) || upload_vec(ctx, &x.m_tbase, tbase) ||
-          upload_vec(ctx, &x.m_ent, ent) || upload_weights(ctx, &x.m_w, w))
-        return fail(ctx, DRN_E_NOMEM, "exchange list upload failed");
-      if (turned && (upload_vec(ctx, &x.m_et, et) || upload_weights(ctx, &x.m_turn, turns)))
-        return fail(ctx, DRN_E_NOMEM, "exchange list upload failed");
-    }
-    return DRN_OK;
+    return upload_multi(ctx, x, order, turns);
   };
   int rc;
   if ((rc = upload_lists(ctx->xfull, false)) || (rc = upload_lists(ctx->xpart, true))) return rc;
   ctx->have_exchange = !ctx->xfull.single.empty() || ctx->xfull.multi_n > 0;
+  ctx->xt_dirty = false;
   ctx->n_fused = n_fused;
   HIPCHK(ctx, hipMemcpy(ctx->d_pd, ctx->pd_host.data(), ctx->pd_host.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
   const std::vector<std::vector<int>> chains = push_chains(ctx, push_pairs);
@@ -2043,7 +2024,135 @@ int drn_exchange_commit(drn_ctx* ctx) {
       if ((rc = build_box(ctx, rk, chains, ctx->box_rk, 3))) return rc;
     }
   }
-  return build_chain_list(ctx, chains, !push_pairs.empty());
+  if ((rc = build_chain_list(ctx, chains, !push_pairs.empty()))) return rc;
+  return build_ls_exchange(ctx);
+}
+
+// the multi-donor receivers, sorted by their number of entries in bands
+// of 8 (descending), so that the 64 lanes of a wavefront loop over about
+// as many entries each, and within a band by their first donor cell, so
+// that the lanes read neighbouring donor cells: on a 200-patch nested
+// batch 0.356 ms per exchange, against 0.564 sorted by the count alone,
+// 0.387 with bands of 1 and 0.385 by the donor cell alone;
+// wavefront b's entries start at tbase[b], entry q of lane L at + 64 q + L
+static int upload_multi(drn_ctx* ctx, drn_ctx::ExchangeLists& x,
+                        std::vector<std::pair<size_t, const ExchangeReceiver*>>& order,
+                        const std::vector<double>& turns) {
+  auto first_donor = [](const ExchangeReceiver* e) -> uint32_t {
+    return e->second.empty() || e->second[0].idx.empty() ? 0u : e->second[0].idx[0];
+  };
+  std::stable_sort(order.begin(), order.end(), [&](const auto& a, const auto& b) {
+    const size_t ka = (a.first + 7) / 8, kb = (b.first + 7) / 8;
+    if (ka != kb) return ka > kb;
+    return first_donor(a.second) < first_donor(b.second);
+  });
+  std::vector<uint32_t> rec, cnt, tbase, ent, et;
+  std::vector<double> w;
+  const bool turned = !turns.empty();
+  for (size_t b = 0; b < order.size(); b += 64) {
+    const size_t nb = std::min<size_t>(64, order.size() - b);
+    size_t emax = 0;
+    for (size_t L = 0; L < nb; ++L) emax = std::max(emax, order[b + L].first);
+    if (ent.size() + 64 * emax > 0xffffffffu) return fail(ctx, DRN_E_RANGE, "exchange lists exceed 2^32 entries");
+    tbase.push_back((uint32_t)ent.size());
+    ent.resize(ent.size() + 64 * emax, 0u);
+    w.resize(ent.size(), 0.0);
+    if (turned) et.resize(ent.size(), 0u);
+    for (size_t L = 0; L < nb; ++L) {
+      const auto& e = *order[b + L].second;
+      rec.push_back(e.first);
+      size_t q = 0;
+      for (const auto& g : e.second) {
+        for (size_t s2 = 0; s2 < g.idx.size(); ++s2, ++q) {
+          const size_t at = tbase.back() + 64 * q + L;
+          if (g.idx[s2] & 0x80000000u) return fail(ctx, DRN_E_RANGE, "donor cell index beyond 2^31");
+          ent[at] = g.idx[s2] | (s2 + 1 == g.idx.size() ? 0x80000000u : 0u);
+          w[at] = g.w[s2];
+          if (turned && s2 + 1 == g.idx.size()) et[at] = (uint32_t)g.turn;
+        }
+      }
+      cnt.push_back((uint32_t)q);
+    }
+  }
+  if (!rec.empty()) {
+    x.multi_n = (uint32_t)rec.size();
+    if (upload_vec(ctx, &x.m_rec, rec) || upload_vec(ctx, &x.m_cnt, cnt) || upload_vec(ctx, &x.m_tbase, tbase) ||
+        upload_vec(ctx, &x.m_ent, ent) || upload_weights(ctx, &x.m_w, w))
+      return fail(ctx, DRN_E_NOMEM, "exchange list upload failed");
+    if (turned && (upload_vec(ctx, &x.m_et, et) || upload_weights(ctx, &x.m_turn, turns)))
+      return fail(ctx, DRN_E_NOMEM, "exchange list upload failed");
+  }
+  return DRN_OK;
+}
+
+// xls: the receivers that a level-set fill can change the exchange of.  After an
+// exchange and a fill the others already hold what another exchange would write
+// (donors are never receivers), so the exchange before the next stage copies
+// these only.  All of them go through the multi-donor list, in one launch.
+static int build_ls_exchange(drn_ctx* ctx) {
+  free_lists(ctx->xls);
+  ctx->exch_ls_buf = -1;
+  ctx->xls_ok = false;
+  if (ctx->xt_dirty || ctx->lt_dirty) return DRN_OK;
+  if (!ctx->have_exchange || ctx->lt.empty()) return DRN_OK;
+  std::vector<bool> filled(ctx->vstride, false);
+  for (const auto& kv : ctx->lt)
+    for (int64_t c : kv.second.cells) filled[ctx->offs[kv.first] + (uint64_t)c] = true;
+  std::vector<double> turns;
+  std::vector<ExchangeReceiver> list;
+  for (const auto& kv : ctx->xt) {
+    const int p = kv.first;
+    const ExchangeTables& t = kv.second;
+    std::map<int64_t, size_t> at;  // touched receiver -> its place in `list`
+    auto touch = [&](int64_t r) {
+      if (at.emplace(r, list.size()).second) list.push_back({(uint32_t)(ctx->offs[p] + (uint64_t)r), {}});
+    };
+    auto each = [&](auto&& f) {
+      for (size_t d = 0; d < t.donor_patch.size(); ++d) {
+        const int64_t nrec = t.donor_info[4 * d], stride = t.donor_info[4 * d + 1], r0 = t.donor_info[4 * d + 2],
+                      w0 = t.donor_info[4 * d + 3];
+        for (int64_t ll = 0; ll < nrec; ++ll) f(d, t.rec_concat[r0 + ll], w0 + ll * stride, stride);
+      }
+    };
+    for (int64_t r : t.rec_unique)
+      if (filled[ctx->offs[p] + (uint64_t)r]) touch(r);
+    each([&](size_t d, int64_t r, int64_t a, int64_t stride) {
+      const uint64_t off = ctx->offs[t.donor_patch[d]];
+      for (int64_t q = a; q < a + stride; ++q)
+        if (filled[off + (uint64_t)t.donor_index[q]]) {
+          touch(r);
+          return;
+        }
+    });
+    if (at.empty()) continue;
+    std::vector<int> turn_of(t.donor_patch.size(), 0);
+    for (size_t d = 0; d < t.donor_patch.size(); ++d)
+      if (!t.turn.empty() && !is_identity_turn(&t.turn[9 * d])) {
+        turns.insert(turns.end(), t.turn.begin() + 9 * d, t.turn.begin() + 9 * (d + 1));
+        turn_of[d] = (int)(turns.size() / 9);
+      }
+    each([&](size_t d, int64_t r, int64_t a, int64_t stride) {
+      const auto it = at.find(r);
+      if (it == at.end()) return;
+      DonorGroup g;
+      g.stride = (int)stride;
+      g.turn = turn_of[d];
+      for (int64_t q = a; q < a + stride; ++q) {
+        g.idx.push_back((uint32_t)(ctx->offs[t.donor_patch[d]] + (uint64_t)t.donor_index[q]));
+        g.w.push_back(t.donor_weight[q]);
+      }
+      list[it->second].second.push_back(std::move(g));
+    });
+  }
+  std::vector<std::pair<size_t, const ExchangeReceiver*>> order;
+  for (const auto& e : list) {
+    size_t n = 0;
+    for (const auto& g : e.second) n += g.idx.size();
+    order.push_back({n, &e});
+  }
+  const int rc = upload_multi(ctx, ctx->xls, order, turns);
+  ctx->xls_ok = rc == DRN_OK;
+  return rc;
 }
 
 int drn_set_exchange_fusion(drn_ctx* ctx, int on) {
@@ -2086,6 +2195,7 @@ int drn_levelset_set(drn_ctx* ctx, int patch, int64_t n, const int64_t* cells, c
   for (int64_t a = 0; a < 8 * n; ++a)
     if (t.donors[a] < 0 || t.donors[a] >= nc) return fail(ctx, DRN_E_RANGE, "mirror donor outside patch");
   ctx->lt[patch] = std::move(t);
+  ctx->lt_dirty = true;
   return DRN_OK;
 }
 
@@ -2107,8 +2217,10 @@ int drn_levelset_commit(drn_ctx* ctx) {
     w.insert(w.end(), t.weights.begin(), t.weights.end());
   }
   ctx->ls_n = (uint32_t)cells.size();
-  if (ctx->ls_n == 0) return DRN_OK;
+  ctx->lt_dirty = false;
   int rc;
+  if ((rc = build_ls_exchange(ctx))) return rc;
+  if (ctx->ls_n == 0) return DRN_OK;
   if ((rc = upload_vec(ctx, &ctx->ls_cells, cells)) || (rc = upload_vec(ctx, &ctx->ls_donors, donors)) ||
       (rc = upload_weights(ctx, &ctx->ls_nrm, nrm)) || (rc = upload_weights(ctx, &ctx->ls_w, w)))
     return rc;
@@ -2150,7 +2262,10 @@ int drn_rk_graph_run(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, 
   int rc;
   // A replay starts from an exchanged state, so that the captured steps may
   // skip the leading exchange as drn_rk_step does; it runs eagerly when needed.
-  if (ctx->exch_buf != ctx->map[0]) {
+  // (with a level-set fill every captured step starts with the exchange of the
+  // receivers the fill touched, so a buffer in that state will do)
+  const bool post = ctx->ls_n > 0;
+  if (ctx->exch_buf != ctx->map[0] && !(post && ctx->exch_ls_buf == ctx->map[0])) {
     if ((rc = do_exchange(ctx, ctx->map[0]))) return rc;
   }
   // A step permutes the three buffers; the steps until the map returns to the
@@ -2186,17 +2301,28 @@ int drn_rk_graph_run(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, 
       // graphs of another step size or other coefficients are not replayed again
       if (!ctx->graphs.empty() && (ctx->graphs[0].dt != dt || ctx->graphs[0].alpha != al)) drop_graph(ctx);
       const bool was_timing = ctx->timing;
-      const int exch0 = ctx->exch_buf;
+      const int exch0 = ctx->exch_buf, exch_ls0 = ctx->exch_ls_buf;
+      if (post) {
+        ctx->exch_buf = -1;
+        ctx->exch_ls_buf = map0[0];
+      }
       ctx->timing = false;
       hipGraph_t graph;
-      HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+      const hipError_t eb = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
+      if (eb != hipSuccess) {
+        ctx->timing = was_timing;
+        ctx->exch_buf = exch0;
+        ctx->exch_ls_buf = exch_ls0;
+        return fail(ctx, DRN_E_HIP, std::string("graph capture: ") + hipGetErrorString(eb));
+      }
       rc = DRN_OK;
       for (int s = 0; s < cyc && rc == DRN_OK; ++s) rc = do_rk_step(ctx, dt, n_alpha, alpha, DRN_LAUNCH_BATCHED);
       hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
-      const int exch_end = ctx->exch_buf;
+      const int exch_end = ctx->exch_buf, exch_ls_end = ctx->exch_ls_buf;
       ctx->timing = was_timing;
       memcpy(ctx->map, map0, sizeof(map0));
       ctx->exch_buf = exch0;
+      ctx->exch_ls_buf = exch_ls0;
       if (rc) {
         if (e == hipSuccess) (void)hipGraphDestroy(graph);
         return rc;
@@ -2208,6 +2334,7 @@ int drn_rk_graph_run(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, 
       g.alpha = al;
       g.steps = cyc;
       g.exch_end = exch_end;
+      g.exch_ls_end = exch_ls_end;
       g.exec = nullptr;
       e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
       (void)hipGraphDestroy(graph);
@@ -2219,6 +2346,7 @@ int drn_rk_graph_run(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, 
     for (; done + cyc <= n_steps; done += cyc) {
       HIPCHK(ctx, hipGraphLaunch(g.exec, ctx->stream));
       ctx->exch_buf = g.exch_end;
+      ctx->exch_ls_buf = g.exch_ls_end;
     }
   }
   // the remainder runs eagerly and advances the map
@@ -2455,7 +2583,7 @@ int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
     const bool push = push_active(ctx, launch);
     auto trial = [&]() {
       int r = do_stage(ctx, ctx->map[0], ctx->map[1], ctx->map[2], 0.0, launch, push, true);
-      return r ? r : do_exchange(ctx, ctx->map[2], push);
+      return r ? r : do_exchange(ctx, ctx->map[2], push ? X_PART : X_FULL);
     };
     rc = trial();  // warm-up
     if (rc) break;
