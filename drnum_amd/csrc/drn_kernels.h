@@ -1573,6 +1573,207 @@ __device__ __forceinline__ void stage_box_item(const PatchDev* __restrict__ pds,
   }
 }
 
+// The box's positions marched over the planes [i0, i1) of an item: each x face
+// and x slope is formed once and carried to the next plane (4 face evaluations
+// and 5 slopes per cell), and the neighbours on the y and z axes come from a
+// tile of the plane in LDS: the cells from two rows below the workgroup's first
+// position to two rows above its last, copied there directly 16 bytes per lane
+// while the plane before is worked on.  Two tiles of N4 x 16 bytes per variable,
+// each an object of its own so that reads of one do not wait for the copies into
+// the other.  NW wavefronts per workgroup.
+// What bounds it: the box kernel's loads take 0.42 of its 0.47 ms on a 64-patch
+// jet of 19.2 M FP32 cells, most of it the stencil's rows and planes coming from
+// L2 again and again.  The same cells read and written in this form take 0.26 ms
+// (a copy of the three fields' bytes 0.21).  The kernel takes 0.375 ms (0.445
+// the box kernel): at 96 VGPRs, 5 wavefronts per SIMD (103 uncapped, 4 per SIMD:
+// 8 % slower), the VALU is the larger part.
+template <typename T, int RECON, int LIM, bool FAST, int N4, int NW>
+struct Sweep {
+  static_assert(sizeof(T) == 4, "the tiles hold 4-byte values");
+  typedef T Tile[5][N4 * 4];
+  const PatchDev& P;
+  const int ni, nj, nk, njk, lane, wv;
+  const T* src;
+  const uint64_t vs;
+  int j, k, lo, hi;
+  bool in, own, hy_m, hy_p, hz_m, hz_p;
+  uint32_t sx, g;  // plane stride and the cell's index in the variable array, in cells
+  T dx, dy, dz, Ax, Ay, Az, pf;
+  T u[5], un[5], xl[5], res[5];
+
+  // start the copy of plane i's tile
+  __device__ __forceinline__ void fetch(int i, Tile& tile) const {
+    const uint32_t first = P.off + (uint32_t)i * (uint32_t)njk;
+    const uint32_t a = (first + (uint32_t)lo) & ~3u;
+    const int n4 = (int)((first + (uint32_t)hi - a + 3) >> 2), per = (n4 + 63) >> 6;
+    for (int q = wv; q < 5 * per; q += NW) {
+      const int v = q / per, b = (q - v * per) * 64;
+      if (b + lane < n4)
+        __builtin_amdgcn_global_load_lds(
+            (__attribute__((address_space(1))) void*)(src + (uint64_t)v * vs + a + 4u * (uint32_t)(b + lane)),
+            (__attribute__((address_space(3))) void*)&tile[v][4 * b], 16, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void cell(uint32_t c, T* x) const {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) x[v] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(src + (uint64_t)v * vs) + c * 4u);
+  }
+  // one plane: its tile is complete in `tile`; `next` is free
+  __device__ __forceinline__ void plane(int i, int i1, Tile& tile, Tile& next, const T* base, T* dst, int push) {
+    if (i + 1 < i1) fetch(i + 1, next);
+    T uf[5], fyp[5], none[5];
+    cell(i + 2 < ni ? g + 2 * sx : (i + 1 < ni ? g + sx : g), uf);
+    const uint32_t first = P.off + (uint32_t)i * (uint32_t)njk;
+    const int l = (int)(g - ((first + (uint32_t)lo) & ~3u));
+    auto at = [&](int d, T* x) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) x[v] = tile[v][l + d];
+    };
+    zero5(fyp);
+    if (nj > 2 && own) {
+      T m[5], p[5], o[5], lo_[5], hi_[5];
+      at(hy_m ? -nk : 0, m);
+      at(hy_p ? nk : 0, p);
+      side_states<T, RECON, LIM, FAST, true, true>(m, u, p, hy_m, hy_p, lo_, hi_);
+      if (hy_m) {
+        T mm[5];
+        at(j >= 2 ? -2 * nk : -nk, mm);
+        side_states<T, RECON, LIM, FAST, false, true>(mm, m, u, j >= 2, true, none, o);
+        const FaceFlux<T> F = face_flux_x<T, FAST, 1>(o, lo_, Ay);
+        T f[5];
+        F.template set<1>(f);
+        F.add(f, res);
+      }
+      if (hy_p) {
+        T pp[5];
+        at(j + 2 < nj ? 2 * nk : nk, pp);
+        side_states<T, RECON, LIM, FAST, true, false>(u, p, pp, true, j + 2 < nj, o, none);
+        face_flux_x<T, FAST, 1>(hi_, o, Ay).template set<1>(fyp);
+      }
+    }
+    T ub[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) ub[v] = ldv<T>(reinterpret_cast<const char*>(base + (uint64_t)v * vs), g * 4u);
+    if (nk > 2) {
+      T m[5], p[5], lo_[5], hi_[5], f[5], o[5];
+      at(hz_m ? -1 : 0, m);
+      at(hz_p ? 1 : 0, p);
+      side_states<T, RECON, LIM, FAST, true, true>(m, u, p, hz_m, hz_p, lo_, hi_);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) o[v] = __shfl_up(hi_[v], 1, 64);
+      zero5(f);
+      if (in && k > P.ka) {
+        const FaceFlux<T> F = face_flux_x<T, FAST, 2>(o, lo_, Az);
+        F.template set<2>(f);
+        F.add(f, res);
+      }
+#pragma unroll
+      for (int v = 0; v < 5; ++v) o[v] = __shfl_down(f[v], 1, 64);
+      sub5(res, o);
+    }
+    sub5(res, fyp);
+    T fx[5], lo_[5], hi_[5];
+    side_states<T, RECON, LIM, FAST, true, true>(u, un, uf, true, i + 2 < ni, lo_, hi_);
+    zero5(fx);
+    if (ni > 2 && i + 1 < ni) face_flux_x<T, FAST, 0>(xl, lo_, Ax).template set<0>(fx);
+    sub5(res, fx);
+    T nv[5];
+    if (own) add_walls<T, FAST>(P, i, j, k, u, dx, dy, dz, res);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) nv[v] = ub[v] + pf * res[v];
+    // the next tile is there, and every wavefront is done with this one; the
+    // stores go out after that wait
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+    if (own) {
+      bool store = true;
+      if (push) {
+        // the fused exchange of the z-face seek layers, as in stage_cell_item
+        for (int s = 0; s < P.nrecv_box; ++s) store = store && !in_box(P.recv[s], i, j, k);
+        for (int s = 0; s < P.npush; ++s) {
+          if (in_box(P.push[s], i, j, k)) {
+            const uint32_t tb =
+                ((uint32_t)P.push_base[s] + (uint32_t)i * P.push_si[s] + (uint32_t)j * P.push_sj[s] + (uint32_t)k) * 4u;
+#pragma unroll
+            for (int v = 0; v < 5; ++v)
+              *reinterpret_cast<T*>(reinterpret_cast<char*>(dst + (uint64_t)v * vs) + tb) = T(0) + nv[v];
+          }
+        }
+      }
+      if (store) {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) *reinterpret_cast<T*>(reinterpret_cast<char*>(dst + (uint64_t)v * vs) + g * 4u) = nv[v];
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      u[v] = un[v];
+      un[v] = uf[v];
+      xl[v] = hi_[v];
+      res[v] = fx[v];
+    }
+    g += sx;
+  }
+};
+
+template <typename T, int RECON, int LIM, bool FAST, int N4, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 5 : 4, NW == 4 ? 5 : 4))) void k_stage_sweep(
+    const PatchDev* __restrict__ pds, const TileMarch* __restrict__ tiles, const T* __restrict__ src, const T* base,
+    T* dst, uint64_t vs, T factor, int push) {
+  typedef Sweep<T, RECON, LIM, FAST, N4, NW> S;
+  __shared__ __align__(16) typename S::Tile t0;
+  __shared__ __align__(16) typename S::Tile t1;
+  const TileMarch t = tiles[blockIdx.x];
+  const PatchDev& P = pds[t.patch];
+  const int lane = (int)(threadIdx.x & 63), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  S s{P, P.ni, P.nj, P.nk, P.njk, lane, wv, src, vs};
+  const int pitch = P.kb - P.ka;
+  auto cell_of = [&](int q) {  // the cell of a position within its plane
+    const int qq = q < 0 ? 0 : (q < P.npos ? q : P.npos - 1);
+    return (P.box.j0 + qq / pitch) * P.nk + P.ka + qq % pitch;
+  };
+  // the tile: two rows and one cell beyond the workgroup's positions
+  const int c_lo = cell_of(t.c0 - 1) - 2 * P.nk - 1, c_hi = cell_of(t.c0 + 62 * NW) + 2 * P.nk + 2;
+  s.lo = c_lo < 0 ? 0 : c_lo;
+  s.hi = c_hi < P.njk ? c_hi : P.njk;
+  const int q = t.c0 + 62 * wv + lane - 1;
+  const int c = cell_of(q);
+  s.j = c / P.nk;
+  s.k = c - s.j * P.nk;
+  s.in = q >= 0 && q < P.npos;
+  s.own = s.in && lane >= 1 && lane <= 62 && s.k >= P.box.k0 && s.k < P.box.k1;
+  s.hy_m = s.j >= 1;
+  s.hy_p = s.j + 1 < P.nj;
+  s.hz_m = s.k >= 1;
+  s.hz_p = s.k + 1 < P.nk;
+  s.sx = (uint32_t)P.njk;
+  s.g = P.off + (uint32_t)t.i0 * (uint32_t)P.njk + (uint32_t)c;
+  s.dx = T(P.dx), s.dy = T(P.dy), s.dz = T(P.dz);
+  s.Ax = s.dy * s.dz, s.Ay = s.dx * s.dz, s.Az = s.dx * s.dy;
+  s.pf = factor / (s.dx * s.dy * s.dz);
+  s.fetch(t.i0, t0);
+  // the x face below the first plane and the state at its upper face
+  {
+    T um[5], umm[5], lo_[5], o[5], none[5];
+    s.cell(s.g, s.u);
+    s.cell(t.i0 + 1 < P.ni ? s.g + s.sx : s.g, s.un);
+    s.cell(t.i0 >= 1 ? s.g - s.sx : s.g, um);
+    s.cell(t.i0 >= 2 ? s.g - 2 * s.sx : (t.i0 >= 1 ? s.g - s.sx : s.g), umm);
+    side_states<T, RECON, LIM, FAST, true, true>(um, s.u, s.un, t.i0 >= 1, t.i0 + 1 < P.ni, lo_, s.xl);
+    zero5(s.res);
+    if (P.ni > 2 && t.i0 > 0) {
+      side_states<T, RECON, LIM, FAST, false, true>(umm, um, s.u, t.i0 >= 2, true, none, o);
+      face_flux_x<T, FAST, 0>(o, lo_, s.Ax).template set<0>(s.res);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the first tile
+  __syncthreads();
+  for (int i = t.i0; i < t.i1; i += 2) {
+    s.plane(i, t.i1, t0, t1, base, dst, push);
+    if (i + 1 < t.i1) s.plane(i + 1, t.i1, t1, t0, base, dst, push);
+  }
+}
+
 template <typename T, int RECON, int LIM, bool FAST, int XP>
 __global__ __launch_bounds__(256) void k_stage_box(const PatchDev* __restrict__ pds, const TileCell* __restrict__ tiles,
                                                    const T* __restrict__ src, const T* base, T* dst, uint64_t vs,

@@ -23,6 +23,7 @@ namespace {
 
 constexpr int NBUF = 3;
 constexpr int ALIGN_CELLS = 64;
+constexpr int kSweepN4[2] = {168, 328};  // tile sizes of the sweep kernel over 4 and 8 wavefronts
 constexpr int kRedBlocksPerCu = 8;  // a full device of 256-thread workgroups
 
 struct ExchangeTables {
@@ -159,6 +160,7 @@ struct drn_ctx {
   PatchDev* d_pd_rk = nullptr;
   int n_dead_faces = 0;
   const PatchDev* pd_stage = nullptr;  // the descriptors of the stage being launched
+  int sweep_waves = 4;                 // wavefronts per workgroup of the sweep being launched
   std::vector<TileCell> tiles;
   std::vector<int> tile_first;  // per patch, size np+1
   TileCell* d_tiles = nullptr;
@@ -188,6 +190,16 @@ struct drn_ctx {
     std::vector<int> first;  // per patch, size np+1 (into d_pp)
     TileCell *d = nullptr, *d_pp = nullptr;  // both in XCD segments
   } box[2], box_rk[3];
+  // items of the sweep kernel over the boxes of the RK step's descriptors, for
+  // one length of the plane range; waves: wavefronts per workgroup
+  struct SweepList {
+    int len = 0, n = 0, waves = 4;
+    std::vector<int> first;
+    TileMarch *d = nullptr, *d_pp = nullptr;
+  } sweep[2];  // per launch form
+  std::vector<PatchDev> rk_host;          // d_pd_rk as uploaded (empty: none)
+  int64_t sweep_waves_all = 0;            // wavefronts of the batched 8-plane sweep list (0: none)
+  std::vector<std::vector<int>> chains;   // patches joined by fused pushes
   std::vector<TileCell> tx2;
   std::vector<int> tx2_first;
   TileCell* d_tx2 = nullptr;
@@ -377,6 +389,7 @@ enum {
   K_CELLXS2 = 13,  // the z-shared cell kernel over 2 planes per item, x faces shared through LDS
   K_CELLXS4 = 14,  // the same over 4 planes per item
   K_BOX1 = 15,     // one thread per cell of the patch's box, one plane per item
+  K_SWEEP = 17,    // the box's positions marched over a range of planes (FP32 fast arithmetic, RK step; else K_BOX4)
   K_BOX4 = 16      // the same over 4 planes per item, x faces shared through LDS
 };
 struct TilingChoice {
@@ -397,9 +410,9 @@ static const TilingChoice kTilings[] = {
     {0, 2, K_CELLZ},   {0, 1, K_XM},         {32, 1, K_XM},    {16, 1, K_XM},    {8, 1, K_XM},
     {0, 1, K_XM8},     {16, 1, K_XM8},       {0, 1, K_XM7},    {16, 1, K_XM7},   {0, 1, K_XML},
     {16, 1, K_XML},    {8, 1, K_XML},        {0, 2, K_CELLXS4}, {0, 1, K_CELLXS4}, {0, 2, K_CELLXS2},
-    {0, 1, K_CELLXS2}, {0, 2, K_BOX1},      {0, 2, K_BOX4}};
+    {0, 1, K_CELLXS2}, {0, 2, K_BOX1},      {0, 2, K_BOX4},   {8, 2, K_SWEEP}};
 static const int kNumTilings = sizeof(kTilings) / sizeof(kTilings[0]);
-static const int kBoxOnePlane = 51, kBoxFourPlanes = 52;
+static const int kBoxOnePlane = 51, kBoxFourPlanes = 52, kSweep8 = 53;
 
 // the column kernel covers the fast MUSCL forms with a symmetric limited slope
 static bool column_capable(const drn_ctx* ctx);
@@ -461,7 +474,16 @@ static void launch_range(drn_ctx* ctx, int kind, const void* tiles, int ntiles, 
                                        kind == K_CELL_SLOPE);
   else if (kind == K_WTILE)
     launch_wtile_t<T, RECON, LIM, FAST>(ctx, (const TileWave*)tiles, ntiles, src, base, dst, factor);
-  else if (kind == K_BOX1 || kind == K_BOX4) {
+  else if (kind == K_SWEEP) {
+    if constexpr (FAST && sizeof(T) == 4) {
+      const bool wide = ctx->sweep_waves == 8;
+      const auto kern = wide ? k_stage_sweep<T, RECON, LIM, FAST, kSweepN4[1], 8>
+                             : k_stage_sweep<T, RECON, LIM, FAST, kSweepN4[0], 4>;
+      if (ntiles > 0)
+        hipLaunchKernelGGL(kern, dim3(ntiles), dim3(wide ? 512 : 256), 0, ctx->stream, ctx->pd_stage, (const TileMarch*)tiles, src,
+                           base, dst, ctx->vstride, factor, (int)ctx->push_now);
+    }
+  } else if (kind == K_BOX1 || kind == K_BOX4) {
     if (ntiles > 0) {
       const auto kern = kind == K_BOX1 ? k_stage_box<T, RECON, LIM, FAST, 1> : k_stage_box<T, RECON, LIM, FAST, 4>;
       hipLaunchKernelGGL(kern, dim3(ntiles), dim3(256), 0, ctx->stream, ctx->pd_stage, (const TileCell*)tiles, src, base,
@@ -567,13 +589,20 @@ static bool column_capable(const drn_ctx* ctx) {
 // The box kernel over four planes per item (52) is the fastest or within 6 % of
 // it on every grid measured from 0.3 to 60 M cells in both precisions (64-patch
 // jet, FP32: 0.467 ms per stage and exchange against 0.612 of choice 11 and
-// 0.495 of 49; 27-patch jet, FP64: 0.303 against 0.458 and 0.351 of 48).  Where
-// its items would not give every CU one, the one-plane form (51) spreads the
-// cells over four times as many workgroups: 8 patches of 8^3 cells, FP64, 14.2
-// us against 22.7; 8 patches of 16^3, FP32, 160 items, 9.4 against 9.5.
+// 0.495 of 49; 27-patch jet, FP64: 0.263 against 0.458 of 11), with two
+// exceptions.  Where its items would not give every CU one, the one-plane form
+// (51) spreads the cells over four times as many workgroups: 8 patches of 8^3
+// cells, FP64, 14.2 us against 22.7; 8 patches of 16^3, FP32, 160 items, 9.4
+// against 9.5.  In FP32 fast arithmetic the sweep (53) is faster once its list
+// fills the device (20 wavefronts per CU) about two and a half times, with the
+// state beyond the caches: us per stage and exchange of 52 / 53 on 3.5 M cells
+// (25 wavefronts per CU) 82 / 90, 8.0 M uneven (60) 256 / 255, 8.5 M (60) 214 /
+// 190, 19.2 M (140) 472 / 399, 60 M (230) 1,453 / 1,342.
 static int tiling_of(const drn_ctx* ctx, int launch) {
   const int set = launch == DRN_LAUNCH_BATCHED ? ctx->tiling : ctx->tiling_pp;
   if (set >= 0) return set;
+  const bool fast32 = ctx->prec == DRN_F32 && (ctx->arith < 0 || ctx->arith == DRN_ARITH_FAST);
+  if (launch == DRN_LAUNCH_BATCHED && fast32 && ctx->sweep_waves_all >= 48 * (int64_t)ctx->n_cu) return kSweep8;
   const int n = (ctx->box_rk[1].n > 0 ? ctx->box_rk : ctx->box)[1].n;
   const int np = launch == DRN_LAUNCH_BATCHED ? 1 : std::max(1, (int)ctx->descs.size());
   return n / np < ctx->n_cu ? kBoxOnePlane : kBoxFourPlanes;
@@ -589,6 +618,7 @@ static int effective_kind(const drn_ctx* ctx, int choice) {
   if (k == K_CELL_SLOPE && !column_capable(ctx)) return K_CELL;
   const bool fast32 = ctx->prec == DRN_F32 && (ctx->arith < 0 || ctx->arith == DRN_ARITH_FAST);
   if ((k == K_XM8 || k == K_XM7) && !fast32) return K_XM;
+  if (k == K_SWEEP && !fast32) return K_BOX4;
   return k;
 }
 
@@ -623,9 +653,16 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
     else
       launch_dispatch<T, false>(ctx, kind, tl, n, src, base, dst, factor);
   };
-  const int choice = tiling_of(ctx, launch), kind = effective_kind(ctx, choice);
+  const int choice = tiling_of(ctx, launch);
+  int kind = effective_kind(ctx, choice);
+  const auto& sw = ctx->sweep[launch == DRN_LAUNCH_BATCHED ? 0 : 1];
+  // a stage of its own covers whole patches, and patches whose tiles would be too large have no list
+  if (kind == K_SWEEP && (ctx->pd_stage == ctx->d_pd || sw.n == 0)) kind = K_BOX4;
+  ctx->sweep_waves = sw.waves;
   if (launch == DRN_LAUNCH_BATCHED) {
-    if (kind == K_BOX1 || kind == K_BOX4 || use_box_cells(ctx, kind)) {
+    if (kind == K_SWEEP) {
+      go(kind, sw.d, sw.n);
+    } else if (kind == K_BOX1 || kind == K_BOX4 || use_box_cells(ctx, kind)) {
       const auto& L = box_list(ctx, kind);
       go(kind, L.d, L.n);
     } else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
@@ -654,7 +691,9 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
     for (int p = 0; p < np; ++p) {
       const int m0 = ctx->mt_first[p], mn = ctx->mt_first[p + 1] - m0;
       const int w0 = ctx->wt_first[p], wn = ctx->wt_first[p + 1] - w0;
-      if (kind == K_BOX1 || kind == K_BOX4 || use_box_cells(ctx, kind)) {
+      if (kind == K_SWEEP) {
+        go(kind, sw.d_pp + sw.first[p], sw.first[p + 1] - sw.first[p]);
+      } else if (kind == K_BOX1 || kind == K_BOX4 || use_box_cells(ctx, kind)) {
         const auto& L = box_list(ctx, kind);
         go(kind, L.d_pp + L.first[p], L.first[p + 1] - L.first[p]);
       } else if (kind == K_CELLXS2 || kind == K_CELLXS4) {
@@ -690,7 +729,7 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
 // fused z-face receivers themselves; the other kinds leave them to the exchange.
 static bool push_kind(int kind) {
   return kind == K_CELL || kind == K_CELLZ || kind == K_CELLZP || kind == K_XM || kind == K_XM8 || kind == K_XM7 ||
-         kind == K_XML || kind == K_CELLXS2 || kind == K_CELLXS4 || kind == K_BOX1 || kind == K_BOX4;
+         kind == K_XML || kind == K_CELLXS2 || kind == K_CELLXS4 || kind == K_BOX1 || kind == K_BOX4 || kind == K_SWEEP;
 }
 
 // whether a stage of this launch form fills the fused receivers (and the
@@ -745,8 +784,95 @@ static int chunk_of(const drn_ctx* ctx, int choice) {
   return k == K_COLUMN || k == K_XM || k == K_XM8 || k == K_XM7 || k == K_XML ? 252 : MARCH_BS;
 }
 
+static void free_sweep(drn_ctx::SweepList& L) {
+  dfree(L.d);
+  dfree(L.d_pp);
+  L = drn_ctx::SweepList();
+}
+
+// wavefronts per workgroup of a sweep over the boxes of `pd`: 4, or 8 where four
+// wavefronts' positions would be few beside the rows around them (192^3 cores:
+// 1,391 us per stage and exchange with 4, whose tiles leave 3 workgroups per CU,
+// 1,342 with 8); 0 where a tile would not fit either
+static int sweep_form(const std::vector<PatchDev>& pd) {
+  // 16-byte units of the largest tile: the positions with the gaps between their
+  // rows, two rows on either side, and the cells that 16-byte alignment adds
+  auto units = [&](int waves) {
+    int n4 = 0;
+    for (const PatchDev& P : pd) {
+      if (P.npos == 0) continue;
+      const int pos = 62 * waves + 2, pitch = P.kb - P.ka;
+      const int cells = pos + (pos / pitch + 1) * (P.nk - pitch) + 4 * P.nk + 10;
+      n4 = std::max(n4, std::min(cells, P.njk + 6) / 4 + 1);
+    }
+    return n4;
+  };
+  if (pd.empty()) return 0;
+  return units(4) <= kSweepN4[0] ? 4 : (units(8) <= kSweepN4[1] ? 8 : 0);
+}
+
+// the sweep kernel's list of plane ranges of `len` planes, in the order of the
+// box lists; none where a patch's tile would exceed the kernel's largest
+static int build_sweep(drn_ctx* ctx, int len, drn_ctx::SweepList& L) {
+  free_sweep(L);
+  const std::vector<PatchDev>& pd = ctx->rk_host;
+  const int waves = sweep_form(pd);
+  if (waves == 0) return DRN_OK;
+  auto segment = [](const std::vector<TileMarch>& nat, size_t a, size_t b, std::vector<TileMarch>& out) {
+    const size_t n = b - a, seg = (n + 7) / 8;
+    for (size_t r = 0; r < seg; ++r)
+      for (size_t x = 0; x < 8; ++x)
+        if (x * seg + r < n) out.push_back(nat[a + x * seg + r]);
+  };
+  auto range = [&](int p, int b, std::vector<TileMarch>& out) {
+    const int i0 = pd[p].box.i0 + b * len, i1 = std::min(pd[p].box.i1, i0 + len);
+    for (int c0 = 0; i0 < i1 && c0 < pd[p].npos; c0 += 62 * waves)
+      out.push_back(TileMarch{p, i0, i1, c0});
+  };
+  const int np = (int)pd.size();
+  std::vector<TileMarch> nat, all, pp;
+  for (const auto& ch : ctx->chains) {
+    int nb = 0;
+    for (int p : ch) nb = std::max(nb, (pd[p].box.i1 - pd[p].box.i0 + len - 1) / len);
+    for (int b = 0; b < nb; ++b)
+      for (int p : ch) range(p, b, nat);
+  }
+  segment(nat, 0, nat.size(), all);
+  nat.clear();
+  L.first.assign(np + 1, 0);
+  for (int p = 0; p < np; ++p) {
+    const size_t a = nat.size();
+    L.first[p] = (int)a;
+    for (int b = 0; b * len < pd[p].box.i1 - pd[p].box.i0; ++b) range(p, b, nat);
+    segment(nat, a, nat.size(), pp);
+  }
+  L.first[np] = (int)nat.size();
+  if (all.empty()) return DRN_OK;
+  HIPCHK(ctx, dalloc(&L.d, all.size()));
+  HIPCHK(ctx, dalloc(&L.d_pp, pp.size()));
+  HIPCHK(ctx, hipMemcpy(L.d, all.data(), all.size() * sizeof(TileMarch), hipMemcpyHostToDevice));
+  HIPCHK(ctx, hipMemcpy(L.d_pp, pp.data(), pp.size() * sizeof(TileMarch), hipMemcpyHostToDevice));
+  L.len = len;
+  L.n = (int)all.size();
+  L.waves = waves;
+  return DRN_OK;
+}
+
+// the sweep lists of the choices in effect
+static int update_sweep(drn_ctx* ctx) {
+  for (int f = 0; f < 2; ++f) {
+    const TilingChoice t = kTilings[tiling_of(ctx, f == 0 ? DRN_LAUNCH_BATCHED : DRN_LAUNCH_PER_PATCH)];
+    if (t.kind != K_SWEEP)
+      free_sweep(ctx->sweep[f]);
+    else if (ctx->sweep[f].len != t.irange)
+      if (const int rc = build_sweep(ctx, t.irange, ctx->sweep[f])) return rc;
+  }
+  return DRN_OK;
+}
+
 // build the marching work-lists of the current tiling choices of both launch forms
 static int build_march(drn_ctx* ctx) {
+  if (const int rcs = update_sweep(ctx)) return rcs;
   const int cb = tiling_of(ctx, DRN_LAUNCH_BATCHED), cp = tiling_of(ctx, DRN_LAUNCH_PER_PATCH);
   const TilingChoice tb = kTilings[cb], tp = kTilings[cp];
   const int np = (int)ctx->descs.size();
@@ -1157,6 +1283,7 @@ void drn_ctx_destroy(drn_ctx* ctx) {
     free_box(ctx->box[w]);
   }
   for (auto& L : ctx->box_rk) free_box(L);
+  for (auto& L : ctx->sweep) free_sweep(L);
   dfree(ctx->d_mt_pp);
   dfree(ctx->d_mt_launch);
   dfree(ctx->d_thin_tiles);
@@ -1775,6 +1902,9 @@ int drn_exchange_commit(drn_ctx* ctx) {
   dfree(ctx->d_pd_rk);
   ctx->d_pd_rk = nullptr;
   for (auto& L : ctx->box_rk) free_box(L);
+  ctx->rk_host.clear();
+  ctx->sweep_waves_all = 0;
+  for (auto& L : ctx->sweep) free_sweep(L);
   for (PatchDev& P : ctx->pd_host) {
     P.npush = P.nrecv = P.nrecv_box = 0;
     memset(P.push, 0, sizeof(P.push));
@@ -1955,6 +2085,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
   ctx->n_fused = n_fused;
   HIPCHK(ctx, hipMemcpy(ctx->d_pd, ctx->pd_host.data(), ctx->pd_host.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
   const std::vector<std::vector<int>> chains = push_chains(ctx, push_pairs);
+  ctx->chains = chains;
   // Dead faces: a face with seek layers whose every boundary cell (the layer the
   // face functor acts on, cartesianiterator.h:190-308) is a receiver of the
   // exchange.  In the RK step the exchange after the stage overwrites those
@@ -2022,6 +2153,12 @@ int drn_exchange_commit(drn_ctx* ctx) {
       HIPCHK(ctx, dalloc(&ctx->d_pd_rk, rk.size()));
       HIPCHK(ctx, hipMemcpy(ctx->d_pd_rk, rk.data(), rk.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
       if ((rc = build_box(ctx, rk, chains, ctx->box_rk, 3))) return rc;
+      ctx->rk_host = rk;
+      if (const int waves = sweep_form(rk))
+        for (const PatchDev& P : rk)
+          ctx->sweep_waves_all +=
+              (int64_t)((P.npos + 62 * waves - 1) / (62 * waves)) * waves * ((P.box.i1 - P.box.i0 + 7) / 8);
+      if ((rc = update_sweep(ctx))) return rc;
     }
   }
   if ((rc = build_chain_list(ctx, chains, !push_pairs.empty()))) return rc;

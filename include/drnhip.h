@@ -328,8 +328,13 @@ int drn_post_variables(drn_ctx* ctx, int field, int patch, int mask, double ref_
  *       drn_rk_step and drn_rk_graph_run each patch's list covers only the box of
  *       its cells that are no exchange receivers (the exchange after the stage
  *       writes those), and the z slopes of a row are formed once per cell.
- * Until a choice is set or autotuned, a rule on the size of the grid picks 51 or
- * 52; drn_get_tiling returns the choice in effect. */
+ * 53    the sweep: the box's positions marched over 8 planes per work item,
+ *       each x face and x slope formed once, the y and z neighbours in an LDS
+ *       tile of the plane that is copied there while the plane before is worked
+ *       on (FP32 fast arithmetic inside drn_rk_step and drn_rk_graph_run, patches
+ *       of up to about 195 cells along z; otherwise 52).
+ * Until a choice is set or autotuned, a rule on the size of the grid picks 51, 52
+ * or 53; drn_get_tiling returns the choice in effect. */
 int drn_num_tilings(void);
 int drn_set_tiling(drn_ctx* ctx, int launch, int choice);
 int drn_get_tiling(const drn_ctx* ctx, int launch);

@@ -1,5 +1,6 @@
-"""The box kernel (tiling choices 51 and 52): one thread per cell of the patch's
-box, which in the RK step leaves out the planes, rows and z layers whose cells
+"""The box kernel (tiling choices 51 and 52) and the sweep over the same positions
+(53, FP32 fast arithmetic in the RK step): one thread per cell of the patch's box,
+which in the RK step leaves out the planes, rows and z layers whose cells
 are all exchange receivers.  Against the oracle where its lanes, planes and
 boxes can go wrong: row lengths around its 62 positions per wavefront, plane
 counts around its 4 planes per item, whole patches (drn_stage alone), thin
@@ -19,7 +20,7 @@ from test_gpu_thin import SHAPES, thin
 pytestmark = pytest.mark.gpu
 
 B, PP = hip.DRN_LAUNCH_BATCHED, hip.DRN_LAUNCH_PER_PATCH
-CHOICES = (51, 52)
+CHOICES = (51, 52, 53)
 
 
 def wave(nx, zc, bc=None):
@@ -40,7 +41,8 @@ def wave(nx, zc, bc=None):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("nx,zc", [(3, 2), (4, 29), (5, 59), (6, 60), (7, 61), (8, 62), (4, 63), (5, 124)])
+@pytest.mark.parametrize("nx,zc", [(3, 2), (4, 29), (5, 59), (6, 60), (7, 61), (8, 62), (4, 63), (5, 124),
+                                   (9, 70), (19, 65), (3, 197)])
 @pytest.mark.parametrize("walls", [False, True])
 def test_lanes_planes_and_rows(gpu, dtype, nx, zc, walls):
     w = wave(nx, zc, [configs.BC_TRANSMISSIVE, configs.BC_SLIP] * 3 if walls else None)
@@ -143,7 +145,8 @@ def test_boxes_change_no_bit(gpu, dtype, make_w):
     in FP32 fast arithmetic also the cell-per-thread kernel (choice 11)."""
     w = make_w()
     ref, _ = run_fused(w, dtype, False, 51, B)
-    forms = [(True, 51, B), (True, 52, B), (True, 51, PP), (True, 52, PP), (False, 52, B)]
+    forms = [(True, 51, B), (True, 52, B), (True, 51, PP), (True, 52, PP), (False, 52, B), (True, 53, B),
+             (True, 53, PP)]
     if dtype == np.float32:
         forms.append((True, 11, B))
     for fuse, choice, launch in forms:
