@@ -3268,24 +3268,36 @@ __global__ __launch_bounds__(256) void k_exchange_multi(uint32_t n, const uint32
 // level-set fill: mirror gather into scratch, then the slip reflection
 // ---------------------------------------------------------------------------
 
+// Eight lanes per layer cell, one mirror donor each: the eight index, weight and
+// value loads of a cell are in flight together and the index and weight loads of
+// a wavefront are contiguous.  The first lane of the eight adds the products in
+// donor order, as one thread did over its eight donors (the fill of 18,900 layer
+// cells, both kernels: 15.6 -> 11.5 us).
 template <typename T>
 __global__ __launch_bounds__(256) void k_ls_access(uint32_t n, const uint32_t* __restrict__ donors,
                                                    const T* __restrict__ w, const T* __restrict__ U, uint64_t vs,
                                                    T* __restrict__ acc) {
 #pragma clang fp contract(off)
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  T a[5];
+  const uint64_t q = (uint64_t)blockIdx.x * 256u + threadIdx.x;  // entry q / 8, donor q % 8
+  const uint64_t e = q >> 3;
+  const bool in = e < n;
+  T t[5], a[5];
+  zero5(t);
   zero5(a);
+  if (in) {
+    const uint64_t d = donors[q];
+    const T ww = w[q];
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const uint64_t d = donors[(uint64_t)e * 8 + s];
-    const T ww = w[(uint64_t)e * 8 + s];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) a[v] += ww * U[v * vs + d];
+    for (int v = 0; v < 5; ++v) t[v] = ww * U[v * vs + d];
   }
 #pragma unroll
-  for (int v = 0; v < 5; ++v) acc[(uint64_t)v * n + e] = a[v];
+  for (int s = 0; s < 8; ++s)
+#pragma unroll
+    for (int v = 0; v < 5; ++v) a[v] += __shfl(t[v], (int)(threadIdx.x & 56u) + s, 64);
+  if (in && (threadIdx.x & 7u) == 0) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) acc[(uint64_t)v * n + e] = a[v];
+  }
 }
 
 // lsobccompressibleeulerop.h:83-144 with the reference's mixed precision

@@ -1085,7 +1085,7 @@ static int do_exchange(drn_ctx* ctx, int pbuf, int which = X_FULL) {
 template <typename T>
 static void launch_ls_t(drn_ctx* ctx, T* U, T relax) {
   const uint32_t n = ctx->ls_n;
-  hipLaunchKernelGGL(k_ls_access<T>, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, ctx->ls_donors,
+  hipLaunchKernelGGL(k_ls_access<T>, dim3((uint32_t)((8 * (uint64_t)n + 255) / 256)), dim3(256), 0, ctx->stream, n, ctx->ls_donors,
                      (const T*)ctx->ls_w, (const T*)U, ctx->vstride, (T*)ctx->ls_acc);
   if (ctx->ls_op == DRN_LS_SWALL)
     hipLaunchKernelGGL(k_ls_operate_swall<T>, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, ctx->ls_cells,
