@@ -995,7 +995,9 @@ static void free_box(drn_ctx::BoxList& L) {
 
 // The work lists over the boxes of `pd` (see BoxList): the
 // planes of a chain's patches side by side, then in 8 contiguous segments, one
-// per XCD; and per patch.  An item covers 62 positions per wavefront.
+// per XCD; and per patch.  An item covers 62 positions per wavefront.  A list
+// gets its counts once both its device copies are complete; without them it is
+// empty.
 static int build_box(drn_ctx* ctx, const std::vector<PatchDev>& pd, const std::vector<std::vector<int>>& chains,
                       drn_ctx::BoxList* lists, int n_lists) {
   auto segment = [](const std::vector<TileCell>& nat, size_t a, size_t b, std::vector<TileCell>& out) {
@@ -1025,20 +1027,21 @@ static int build_box(drn_ctx* ctx, const std::vector<PatchDev>& pd, const std::v
           if (i >= pd[p].box.i0 && i < pd[p].box.i1 && (i - pd[p].box.i0) % xp == 0) plane(p, i, nat);
     }
     segment(nat, 0, nat.size(), all);
-    L.n = (int)all.size();
-    L.first.assign(np + 1, 0);
+    std::vector<int> first(np + 1, 0);
     nat.clear();
     for (int p = 0; p < np; ++p) {
       const size_t a = nat.size();
-      L.first[p] = (int)a;
+      first[p] = (int)a;
       for (int i = pd[p].box.i0; i < pd[p].box.i1; i += xp) plane(p, i, nat);
       segment(nat, a, nat.size(), pp);
     }
-    L.first[np] = (int)nat.size();
+    first[np] = (int)nat.size();
     HIPCHK(ctx, dalloc(&L.d, all.size()));
     HIPCHK(ctx, dalloc(&L.d_pp, pp.size()));
     if (!all.empty()) HIPCHK(ctx, hipMemcpy(L.d, all.data(), all.size() * sizeof(TileCell), hipMemcpyHostToDevice));
     if (!pp.empty()) HIPCHK(ctx, hipMemcpy(L.d_pp, pp.data(), pp.size() * sizeof(TileCell), hipMemcpyHostToDevice));
+    L.n = (int)all.size();
+    L.first = std::move(first);
   }
   return DRN_OK;
 }
@@ -1867,8 +1870,14 @@ static int build_chain_list(drn_ctx* ctx, const std::vector<std::vector<int>>& c
     for (int r = 0; r < seg; ++r)
       for (int x = 0; x < 8; ++x)
         if (x * seg + r < n) out.push_back(nat[x * seg + r]);
-    HIPCHK(ctx, dalloc(dptr, n));
-    HIPCHK(ctx, hipMemcpy(*dptr, out.data(), n * sizeof(TileCell), hipMemcpyHostToDevice));
+    TileCell* d = nullptr;
+    HIPCHK(ctx, dalloc(&d, n));
+    const hipError_t e = hipMemcpy(d, out.data(), n * sizeof(TileCell), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      dfree(d);
+      return fail(ctx, DRN_E_HIP, std::string("chain list: ") + hipGetErrorString(e));
+    }
+    *dptr = d;  // set once it is complete
     return DRN_OK;
   };
   int rc;
@@ -1891,6 +1900,94 @@ static int upload_multi(drn_ctx* ctx, drn_ctx::ExchangeLists& x,
                         const std::vector<double>& turns);
 static int build_ls_exchange(drn_ctx* ctx);
 
+// The RK step's patch descriptors and the work lists over their boxes.
+// Dead faces: a face with seek layers whose every boundary cell (the layer the
+// face functor acts on, cartesianiterator.h:190-308) is a receiver of the
+// exchange.  In the RK step the exchange after the stage overwrites those
+// cells, so the functor's flux there never reaches the state.
+static int build_rk_boxes(drn_ctx* ctx) {
+  std::vector<PatchDev> rk = ctx->pd_host;
+  int dead = 0;
+  bool trimmed = false;
+  for (const auto& kv : ctx->xt) {
+    const int p = kv.first;
+    const drn_patch_desc& d = ctx->descs[p];
+    std::vector<bool> is_rec((size_t)d.ni * d.nj * d.nk, false);
+    for (int64_t r : kv.second.rec_unique) is_rec[(size_t)r] = true;
+    const int n3[3] = {d.ni, d.nj, d.nk};
+    for (int f = 0; f < 6; ++f) {
+      const int a = f >> 1;
+      if (d.seek[f] < 1 || n3[a] <= 2) continue;
+      const int fixed = (f & 1) ? n3[a] - 1 : 0;
+      const int b = (a + 1) % 3, c = (a + 2) % 3;
+      bool all = true;
+      for (int u = 0; u < n3[b] && all; ++u)
+        for (int v = 0; v < n3[c] && all; ++v) {
+          int ijk[3];
+          ijk[a] = fixed;
+          ijk[b] = u;
+          ijk[c] = v;
+          all = is_rec[((size_t)ijk[0] * d.nj + ijk[1]) * d.nk + ijk[2]];
+        }
+      if (all) {
+        rk[p].bc[f] = BC_DEAD;
+        ++dead;
+      }
+    }
+    // The box of the cells that are no receivers, the only ones whose new
+    // state survives that exchange: planes, rows and z layers of receivers
+    // around it are left out of the RK step's box lists.
+    CellBox b{d.ni, 0, d.nj, 0, d.nk, 0};
+    size_t l = 0;
+    for (int i = 0; i < d.ni; ++i)
+      for (int j = 0; j < d.nj; ++j)
+        for (int k = 0; k < d.nk; ++k, ++l) {
+          if (is_rec[l]) continue;
+          b.i0 = std::min(b.i0, i);
+          b.i1 = std::max(b.i1, i + 1);
+          b.j0 = std::min(b.j0, j);
+          b.j1 = std::max(b.j1, j + 1);
+          b.k0 = std::min(b.k0, k);
+          b.k1 = std::max(b.k1, k + 1);
+        }
+    if (b.i1 == 0) b = CellBox{0, 0, 0, 0, 0, 0};
+    trimmed = trimmed || b.i0 > 0 || b.i1 < d.ni || b.j0 > 0 || b.j1 < d.nj || b.k0 > 0 || b.k1 < d.nk;
+    PatchDev& P = rk[p];
+    set_box(P, b);
+    // the receive boxes that meet it come first
+    auto meets = [&](const CellBox& r) {
+      return std::max(r.i0, b.i0) < std::min(r.i1, b.i1) && std::max(r.j0, b.j0) < std::min(r.j1, b.j1) &&
+             std::max(r.k0, b.k0) < std::min(r.k1, b.k1);
+    };
+    if (P.nrecv == 2 && !meets(P.recv[0])) std::swap(P.recv[0], P.recv[1]);
+    P.nrecv_box = 0;
+    while (P.nrecv_box < P.nrecv && meets(P.recv[P.nrecv_box])) ++P.nrecv_box;
+  }
+  ctx->n_dead_faces = dead;
+  if (dead > 0 || trimmed) {
+    HIPCHK(ctx, dalloc(&ctx->d_pd_rk, rk.size()));
+    HIPCHK(ctx, hipMemcpy(ctx->d_pd_rk, rk.data(), rk.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
+    int rc;
+    if ((rc = build_box(ctx, rk, ctx->chains, ctx->box_rk, 3))) return rc;
+    ctx->rk_host = rk;
+    if (const int waves = sweep_form(rk))
+      for (const PatchDev& P : rk)
+        ctx->sweep_waves_all +=
+            (int64_t)((P.npos + 62 * waves - 1) / (62 * waves)) * waves * ((P.box.i1 - P.box.i0 + 7) / 8);
+    if ((rc = update_sweep(ctx))) return rc;
+  }
+  return DRN_OK;
+}
+
+static void free_rk_boxes(drn_ctx* ctx) {
+  dfree(ctx->d_pd_rk);
+  ctx->d_pd_rk = nullptr;
+  for (auto& L : ctx->box_rk) free_box(L);
+  ctx->rk_host.clear();
+  ctx->sweep_waves_all = 0;
+  for (auto& L : ctx->sweep) free_sweep(L);
+}
+
 int drn_exchange_commit(drn_ctx* ctx) {
   if (!ctx) return DRN_E_ARG;
   if (!ctx->laid_out) return fail(ctx, DRN_E_STATE, "drn_layout not called");
@@ -1899,12 +1996,7 @@ int drn_exchange_commit(drn_ctx* ctx) {
   drop_graph(ctx);  // a captured step holds the old lists
   free_exchange(ctx);
   // without receivers no face is dead and every box is the whole patch
-  dfree(ctx->d_pd_rk);
-  ctx->d_pd_rk = nullptr;
-  for (auto& L : ctx->box_rk) free_box(L);
-  ctx->rk_host.clear();
-  ctx->sweep_waves_all = 0;
-  for (auto& L : ctx->sweep) free_sweep(L);
+  free_rk_boxes(ctx);
   for (PatchDev& P : ctx->pd_host) {
     P.npush = P.nrecv = P.nrecv_box = 0;
     memset(P.push, 0, sizeof(P.push));
@@ -2082,86 +2174,16 @@ int drn_exchange_commit(drn_ctx* ctx) {
   if ((rc = upload_lists(ctx->xfull, false)) || (rc = upload_lists(ctx->xpart, true))) return rc;
   ctx->have_exchange = !ctx->xfull.single.empty() || ctx->xfull.multi_n > 0;
   ctx->xt_dirty = false;
-  ctx->n_fused = n_fused;
   HIPCHK(ctx, hipMemcpy(ctx->d_pd, ctx->pd_host.data(), ctx->pd_host.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
-  const std::vector<std::vector<int>> chains = push_chains(ctx, push_pairs);
-  ctx->chains = chains;
-  // Dead faces: a face with seek layers whose every boundary cell (the layer the
-  // face functor acts on, cartesianiterator.h:190-308) is a receiver of the
-  // exchange.  In the RK step the exchange after the stage overwrites those
-  // cells, so the functor's flux there never reaches the state.
-  {
-    std::vector<PatchDev> rk = ctx->pd_host;
-    int dead = 0;
-    bool trimmed = false;
-    for (const auto& kv : ctx->xt) {
-      const int p = kv.first;
-      const drn_patch_desc& d = ctx->descs[p];
-      std::vector<bool> is_rec((size_t)d.ni * d.nj * d.nk, false);
-      for (int64_t r : kv.second.rec_unique) is_rec[(size_t)r] = true;
-      const int n3[3] = {d.ni, d.nj, d.nk};
-      for (int f = 0; f < 6; ++f) {
-        const int a = f >> 1;
-        if (d.seek[f] < 1 || n3[a] <= 2) continue;
-        const int fixed = (f & 1) ? n3[a] - 1 : 0;
-        const int b = (a + 1) % 3, c = (a + 2) % 3;
-        bool all = true;
-        for (int u = 0; u < n3[b] && all; ++u)
-          for (int v = 0; v < n3[c] && all; ++v) {
-            int ijk[3];
-            ijk[a] = fixed;
-            ijk[b] = u;
-            ijk[c] = v;
-            all = is_rec[((size_t)ijk[0] * d.nj + ijk[1]) * d.nk + ijk[2]];
-          }
-        if (all) {
-          rk[p].bc[f] = BC_DEAD;
-          ++dead;
-        }
-      }
-      // The box of the cells that are no receivers, the only ones whose new
-      // state survives that exchange: planes, rows and z layers of receivers
-      // around it are left out of the RK step's box lists.
-      CellBox b{d.ni, 0, d.nj, 0, d.nk, 0};
-      size_t l = 0;
-      for (int i = 0; i < d.ni; ++i)
-        for (int j = 0; j < d.nj; ++j)
-          for (int k = 0; k < d.nk; ++k, ++l) {
-            if (is_rec[l]) continue;
-            b.i0 = std::min(b.i0, i);
-            b.i1 = std::max(b.i1, i + 1);
-            b.j0 = std::min(b.j0, j);
-            b.j1 = std::max(b.j1, j + 1);
-            b.k0 = std::min(b.k0, k);
-            b.k1 = std::max(b.k1, k + 1);
-          }
-      if (b.i1 == 0) b = CellBox{0, 0, 0, 0, 0, 0};
-      trimmed = trimmed || b.i0 > 0 || b.i1 < d.ni || b.j0 > 0 || b.j1 < d.nj || b.k0 > 0 || b.k1 < d.nk;
-      PatchDev& P = rk[p];
-      set_box(P, b);
-      // the receive boxes that meet it come first
-      auto meets = [&](const CellBox& r) {
-        return std::max(r.i0, b.i0) < std::min(r.i1, b.i1) && std::max(r.j0, b.j0) < std::min(r.j1, b.j1) &&
-               std::max(r.k0, b.k0) < std::min(r.k1, b.k1);
-      };
-      if (P.nrecv == 2 && !meets(P.recv[0])) std::swap(P.recv[0], P.recv[1]);
-      P.nrecv_box = 0;
-      while (P.nrecv_box < P.nrecv && meets(P.recv[P.nrecv_box])) ++P.nrecv_box;
-    }
-    ctx->n_dead_faces = dead;
-    if (dead > 0 || trimmed) {
-      HIPCHK(ctx, dalloc(&ctx->d_pd_rk, rk.size()));
-      HIPCHK(ctx, hipMemcpy(ctx->d_pd_rk, rk.data(), rk.size() * sizeof(PatchDev), hipMemcpyHostToDevice));
-      if ((rc = build_box(ctx, rk, chains, ctx->box_rk, 3))) return rc;
-      ctx->rk_host = rk;
-      if (const int waves = sweep_form(rk))
-        for (const PatchDev& P : rk)
-          ctx->sweep_waves_all +=
-              (int64_t)((P.npos + 62 * waves - 1) / (62 * waves)) * waves * ((P.box.i1 - P.box.i0 + 7) / 8);
-      if ((rc = update_sweep(ctx))) return rc;
-    }
+  ctx->n_fused = n_fused;
+  ctx->chains = push_chains(ctx, push_pairs);
+  // without these lists the stages run on whole patches, without the others in
+  // another order or on the full exchange
+  if ((rc = build_rk_boxes(ctx))) {
+    free_rk_boxes(ctx);
+    return rc;
   }
-  if ((rc = build_chain_list(ctx, chains, !push_pairs.empty()))) return rc;
+  if ((rc = build_chain_list(ctx, ctx->chains, !push_pairs.empty()))) return rc;
   return build_ls_exchange(ctx);
 }
 
