@@ -2365,6 +2365,9 @@ int drn_levelset_commit(drn_ctx* ctx) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   free_ls(ctx);
+  free_lists(ctx->xls);
+  ctx->xls_ok = false;
+  ctx->exch_ls_buf = -1;
   std::vector<uint32_t> cells, donors;
   std::vector<double> nrm, w;
   for (auto& kv : ctx->lt) {
@@ -2375,16 +2378,16 @@ int drn_levelset_commit(drn_ctx* ctx) {
     nrm.insert(nrm.end(), t.normals.begin(), t.normals.end());
     w.insert(w.end(), t.weights.begin(), t.weights.end());
   }
-  ctx->ls_n = (uint32_t)cells.size();
-  ctx->lt_dirty = false;
   int rc;
-  if ((rc = build_ls_exchange(ctx))) return rc;
-  if (ctx->ls_n == 0) return DRN_OK;
-  if ((rc = upload_vec(ctx, &ctx->ls_cells, cells)) || (rc = upload_vec(ctx, &ctx->ls_donors, donors)) ||
-      (rc = upload_weights(ctx, &ctx->ls_nrm, nrm)) || (rc = upload_weights(ctx, &ctx->ls_w, w)))
-    return rc;
-  HIPCHK(ctx, hipMalloc(&ctx->ls_acc, (size_t)5 * ctx->ls_n * ctx->esize() + 16));
-  return DRN_OK;
+  if (!cells.empty()) {
+    if ((rc = upload_vec(ctx, &ctx->ls_cells, cells)) || (rc = upload_vec(ctx, &ctx->ls_donors, donors)) ||
+        (rc = upload_weights(ctx, &ctx->ls_nrm, nrm)) || (rc = upload_weights(ctx, &ctx->ls_w, w)))
+      return rc;
+    HIPCHK(ctx, hipMalloc(&ctx->ls_acc, (size_t)5 * cells.size() * ctx->esize() + 16));
+  }
+  ctx->ls_n = (uint32_t)cells.size();  // once the lists are complete: without them there is no fill
+  ctx->lt_dirty = false;
+  return build_ls_exchange(ctx);
 }
 
 int drn_set_levelset_op(drn_ctx* ctx, int op) {

@@ -1,6 +1,6 @@
 """A table commit that runs out of device memory returns an error and leaves a
 context whose steps launch on complete lists only: every device allocation and
-copy of the commit fails once, and the stages after it are looked
+copy of the commit fails once, and the stages, the exchange and the fill after it are looked
 over (CPU: the launches are recorded, not carried out)."""
 import ctypes as C
 
@@ -41,6 +41,9 @@ def _check(calls, np_, n_stage, what):
         patches = np.ctypeslib.as_array(C.cast(tiles, C.POINTER(C.c_int32)), (grid * per // 4,)).reshape(grid, 4)[:, 0]
         assert patches.min() >= 0 and patches.max() < np_, (what, name)
     assert sum(c[1] for c in stages) in n_stage, (what, sum(c[1] for c in stages), n_stage)
+    for name, n, a0, a1 in calls:
+        if name.startswith("k_ls_access"):
+            assert fakedev.fake.fake_is_device(a1), (what, name)
 
 
 def exchange_child():
@@ -80,6 +83,37 @@ def exchange_child():
             assert k > 10
 
 
-@pytest.mark.parametrize("child", ["exchange_child"])
+def levelset_child():
+    from drnum_amd import configs
+
+    fail = fakedev.fake.fake_fail_after
+    w = configs.levelset_spheres(core=16, blocks=(2, 1, 1), n_spheres=1, r_range=(3.0, 3.5))
+    k = 0
+    while True:
+        hg, ctx = _context(w, None, False)
+        hg.upload_exchange(ctx)
+        hg.levelset_spheres(w.spheres, w.ls_inner_layers, 0, w.ls_min_inner_rel)
+        fail(k)
+        failed = False
+        try:
+            hg.upload_levelset(ctx)
+        except Exception:
+            failed = True
+        fail(-1)
+        calls = _step(ctx, w, 0)
+        _check(calls, len(w.patches), {sum(c[1] for c in calls if c[0].startswith("k_stage"))}, k)
+        if failed:
+            hg.upload_levelset(ctx)
+        calls = _step(ctx, w, 0)
+        assert any(c[0].startswith("k_ls_access") for c in calls)
+        _check(calls, len(w.patches), {sum(c[1] for c in calls if c[0].startswith("k_stage"))}, k)
+        ctx.close()
+        if not failed:
+            break
+        k += 1
+    assert k > 4
+
+
+@pytest.mark.parametrize("child", ["exchange_child", "levelset_child"])
 def test_every_allocation_and_copy_may_fail(tmp_path, child):
     run_child(tmp_path, "test_failed_commits", child)
