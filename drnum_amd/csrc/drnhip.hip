@@ -2263,8 +2263,11 @@ static int build_ls_exchange(drn_ctx* ctx) {
     const int p = kv.first;
     const ExchangeTables& t = kv.second;
     std::map<int64_t, size_t> at;  // touched receiver -> its place in `list`
+    // a cell in a donor's receiver list only is written by no exchange
+    std::vector<bool> unique(drn_patch_cells(ctx, p), false);
+    for (int64_t r : t.rec_unique) unique[(size_t)r] = true;
     auto touch = [&](int64_t r) {
-      if (at.emplace(r, list.size()).second) list.push_back({(uint32_t)(ctx->offs[p] + (uint64_t)r), {}});
+      if (unique[(size_t)r] && at.emplace(r, list.size()).second) list.push_back({(uint32_t)(ctx->offs[p] + (uint64_t)r), {}});
     };
     auto each = [&](auto&& f) {
       for (size_t d = 0; d < t.donor_patch.size(); ++d) {
