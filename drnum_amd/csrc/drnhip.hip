@@ -215,6 +215,8 @@ struct drn_ctx {
   double* h_out = nullptr;   // pinned: results of the reductions
   double* d_hout = nullptr;  // its device address
   // hand-over of host buffers: two halves of pinned staging memory, used in turn
+  // by one call at a time (copy_mu: patches may be handed over by several threads)
+  std::mutex copy_mu;
   HostCopier copier;
   char* stage = nullptr;
   size_t stage_half = 0;
@@ -1580,6 +1582,7 @@ static int ensure_stage(drn_ctx* ctx) {
 // Complete on return.
 template <typename E, bool TO_HOST>
 static int host_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
+  std::lock_guard<std::mutex> lock(ctx->copy_mu);
   int rc = ensure_stage(ctx);
   if (rc || total == 0) return rc;
   const uint64_t per = ctx->stage_half / sizeof(E) / 64 * 64, pieces = (total + per - 1) / per;

@@ -1,0 +1,64 @@
+"""drn_patch_upload / drn_patch_download / drn_post_variables beyond the pageable
+buffer on one thread: several threads on one context, and the caller's buffer changed
+right after the call (CPU: k_host_copy is carried out by the stand-in runtime when
+the host waits for it)."""
+import threading
+
+import numpy as np
+import pytest
+
+import fakedev
+from fakedev import run_child
+
+# value counts that divide into 16-byte lanes and not, below and above a staging half of 8 MiB
+SHAPES = [(3, 1, 1), (5, 7, 9), (40, 40, 40), (75, 75, 75), (90, 91, 93)]
+
+
+def _grid(dtype, shapes=SHAPES):
+    from drnum_amd import configs, hip
+
+    ctx = hip.Context(dtype)
+    ctx.set_operator(configs.RECON_UPWIND2, configs.LIM_VANALBADA)
+    for n in shapes:
+        ctx.add_patch(*n, [0] * 6, (1.0, 1.0, 1.0), [configs.BC_SLIP] * 6, np.zeros((6, configs.NPAR)))
+    ctx.layout()
+    return ctx, [np.random.default_rng(7 + p).standard_normal((5, int(np.prod(n)))).astype(dtype)
+                 for p, n in enumerate(shapes)]
+
+
+def pageable_child():
+    for dtype in (np.float32, np.float64):
+        ctx, states = _grid(dtype)
+        for p, U in enumerate(states):
+            a = U.copy()
+            ctx.upload(p, 0, a)
+            a[:] = 0
+        for p, U in enumerate(states):
+            assert np.array_equal(ctx.download(p, 0), U), SHAPES[p]
+        ctx.close()
+
+
+def threads_child():
+    for dtype in (np.float32, np.float64):
+        shapes = [(60, 61, 63), (75, 75, 75), (90, 91, 93), (80, 80, 80)]
+        ctx, states = _grid(dtype, shapes)
+        for _ in range(5):
+            bad = []
+
+            def work(p):
+                ctx.upload(p, 0, states[p])
+                if not np.array_equal(ctx.download(p, 0), states[p]):
+                    bad.append(shapes[p])
+
+            ts = [threading.Thread(target=work, args=(p,)) for p in range(len(shapes))]
+            for t in ts:
+                t.start()
+            for t in ts:
+                t.join()
+            assert not bad, bad
+        ctx.close()
+
+
+@pytest.mark.parametrize("child", ["pageable_child", "threads_child"])
+def test_transfers(tmp_path, child):
+    run_child(tmp_path, "test_transfer_paths", child)
