@@ -1561,30 +1561,44 @@ static int check_field(drn_ctx* ctx, int field) {
   return DRN_OK;
 }
 
-// the staging memory: each half holds the largest patch, at most 8 MiB (60 M FP32
+// The staging memory: each half holds the largest patch, at most 8 MiB (60 M FP32
 // cells in 8 patches up / down, ms: 29 / 38, with halves of 4 MiB 36 / 49, of 1
-// MiB 45 / 77: a piece costs a launch, a wait and a wake-up of the helpers)
-static int ensure_stage(drn_ctx* ctx) {
-  if (ctx->stage) return DRN_OK;
+// MiB 45 / 77: a piece costs a launch, a wait and a wake-up of the helpers).
+// False where no pinned memory is left.
+static bool ensure_stage(drn_ctx* ctx) {
+  if (ctx->stage) return true;
   size_t most = 0;
   for (size_t p = 0; p < ctx->descs.size(); ++p) most = std::max(most, drn_patch_cells(ctx, (int)p));
   const size_t half = std::min<size_t>(8 << 20, (most * 5 * ctx->esize() + 4095) / 4096 * 4096);
-  for (auto& e : ctx->stage_ev)
-    if (!e) HIPCHK(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  HIPCHK(ctx, hipHostMalloc((void**)&ctx->stage, 2 * half, hipHostMallocDefault));
+  bool ok = true;
+  for (auto& e : ctx->stage_ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+  ok = ok && hipHostMalloc((void**)&ctx->stage, 2 * half, hipHostMallocDefault) == hipSuccess;
+  if (!ok) {
+    ctx->stage = nullptr;
+    (void)hipGetLastError();  // the next launch's check must not report it
+    return false;
+  }
   ctx->stage_half = half;
+  return true;
+}
+
+// host_copy without the staging memory: one copy by the runtime per variable
+template <typename E, bool TO_HOST>
+static int direct_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
+  for (uint64_t v = 0; v * n < total; ++v) {
+    E *d = arr + v * vs, *h = (E*)host + v * n;
+    HIPCHK(ctx, hipMemcpyAsync(TO_HOST ? h : d, TO_HOST ? d : h, n * sizeof(E),
+                               TO_HOST ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, ctx->stream));
+  }
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return DRN_OK;
 }
 
-// Copies `total` values between the caller's buffer `host` and the device (the
-// layout of k_host_copy), piece by piece through the staging halves: one half is
-// filled or emptied by the host threads while the device works on the other.
-// Complete on return.
+// host_copy piece by piece through the staging halves: one half is filled or
+// emptied by the host threads while the device works on the other
 template <typename E, bool TO_HOST>
-static int host_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
-  std::lock_guard<std::mutex> lock(ctx->copy_mu);
-  int rc = ensure_stage(ctx);
-  if (rc || total == 0) return rc;
+static int staged_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
+  int rc;
   const uint64_t per = ctx->stage_half / sizeof(E) / 64 * 64, pieces = (total + per - 1) / per;
   constexpr uint32_t M = 16 / sizeof(E);
   auto launch = [&](uint64_t q) -> int {
@@ -1631,6 +1645,18 @@ static int host_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t tot
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
   return DRN_OK;
+}
+
+// Copies `total` values between the caller's buffer `host` and the device (the
+// layout of k_host_copy).  Complete on return.
+template <typename E, bool TO_HOST>
+static int host_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
+  if (total == 0) return DRN_OK;
+  std::lock_guard<std::mutex> lock(ctx->copy_mu);
+  if (!ensure_stage(ctx)) return direct_copy<E, TO_HOST>(ctx, arr, vs, n, total, host);
+  const int rc = staged_copy<E, TO_HOST>(ctx, arr, vs, n, total, host);
+  if (rc) (void)hipStreamSynchronize(ctx->stream);  // the staging memory is free for the next call
+  return rc;
 }
 
 int drn_patch_upload(drn_ctx* ctx, int id, int field, const void* host) {

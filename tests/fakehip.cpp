@@ -25,6 +25,7 @@ std::map<void*, double> event_ms;
 size_t done = 0;                 // operations carried out
 long fail_after = -1;            // device allocations and blocking copies until one fails, -1: none
 int fail_pinned = 0;
+thread_local int last_error = 0;
 std::string journal;
 double clock_ms = 0;
 struct Config {
@@ -189,7 +190,11 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_
   return 0;
 }
 const char* hipGetErrorString(int e) { return e ? "injected" : "none"; }
-int hipGetLastError() { return 0; }
+int hipGetLastError() {
+  const int e = last_error;
+  last_error = 0;
+  return e;
+}
 int hipGetSymbolAddress(void** p, const void*) {
   static char word[64];
   *p = word;
@@ -209,7 +214,7 @@ int hipHostMalloc(void** p, size_t n, unsigned) {
   Lock l(mu);
   if (fail_pinned) {
     *p = nullptr;
-    return 2;
+    return last_error = 2;
   }
   return allocate(pinned, p, n);
 }

@@ -1,5 +1,6 @@
 """drn_patch_upload / drn_patch_download / drn_post_variables beyond the pageable
-buffer on one thread: several threads on one context, and the caller's buffer changed
+buffer on one thread: no pinned
+memory left, several threads on one context, and the caller's buffer changed
 right after the call (CPU: k_host_copy is carried out by the stand-in runtime when
 the host waits for it)."""
 import threading
@@ -38,6 +39,19 @@ def pageable_child():
         ctx.close()
 
 
+def no_pinned_child():
+    for dtype in (np.float32, np.float64):
+        ctx, states = _grid(dtype)
+        fakedev.fake.fake_fail_pinned(1)
+        for p, U in enumerate(states):
+            ctx.upload(p, 0, U)
+        for p, U in enumerate(states):
+            assert np.array_equal(ctx.download(p, 0), U), SHAPES[p]
+        ctx.post_variables(1, ("rho", "p"))
+        fakedev.fake.fake_fail_pinned(0)
+        ctx.close()
+
+
 def threads_child():
     for dtype in (np.float32, np.float64):
         shapes = [(60, 61, 63), (75, 75, 75), (90, 91, 93), (80, 80, 80)]
@@ -59,6 +73,6 @@ def threads_child():
         ctx.close()
 
 
-@pytest.mark.parametrize("child", ["pageable_child", "threads_child"])
+@pytest.mark.parametrize("child", ["pageable_child", "no_pinned_child", "threads_child"])
 def test_transfers(tmp_path, child):
     run_child(tmp_path, "test_transfer_paths", child)
