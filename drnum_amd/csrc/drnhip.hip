@@ -1582,6 +1582,16 @@ static bool ensure_stage(drn_ctx* ctx) {
   return true;
 }
 
+// whether the device can reach `host` itself: pinned, managed or device memory
+static bool reachable(const void* host) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 // host_copy without the staging memory: one copy by the runtime per variable
 template <typename E, bool TO_HOST>
 static int direct_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
@@ -1648,10 +1658,12 @@ static int staged_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t t
 }
 
 // Copies `total` values between the caller's buffer `host` and the device (the
-// layout of k_host_copy).  Complete on return.
+// layout of k_host_copy).  Complete on return.  A buffer that the runtime copies
+// at the link's rate, without a pass of the host over it, is left to it.
 template <typename E, bool TO_HOST>
 static int host_copy(drn_ctx* ctx, E* arr, uint64_t vs, uint64_t n, uint64_t total, void* host) {
   if (total == 0) return DRN_OK;
+  if (reachable(host)) return direct_copy<E, TO_HOST>(ctx, arr, vs, n, total, host);
   std::lock_guard<std::mutex> lock(ctx->copy_mu);
   if (!ensure_stage(ctx)) return direct_copy<E, TO_HOST>(ctx, arr, vs, n, total, host);
   const int rc = staged_copy<E, TO_HOST>(ctx, arr, vs, n, total, host);

@@ -29,3 +29,62 @@ def test_round_trip_is_exact(gpu, dtype):
     rho = ctx.post_variables(7, ("rho",), field=2)["rho"]
     assert np.array_equal(rho, states[7][0])
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_odd_counts_over_several_pieces(gpu, dtype):
+    """the one-value lanes of k_host_copy across variables and reused halves"""
+    ctx = hip.Context(dtype)
+    ctx.set_operator(configs.RECON_UPWIND2, configs.LIM_VANALBADA)
+    for n in ((81, 81, 81), (95, 93, 91)):
+        ctx.add_patch(*n, [0] * 6, (1.0, 1.0, 1.0), [configs.BC_SLIP] * 6, np.zeros((6, configs.NPAR)))
+    ctx.layout()
+    rng = np.random.default_rng(4)
+    states = [rng.standard_normal((5, ctx.patch_cells(p))).astype(dtype) for p in range(2)]
+    for p, U in enumerate(states):
+        ctx.upload(p, 1, U)
+    for p, U in enumerate(states):
+        assert np.array_equal(ctx.download(p, 1), U)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_post_variables_over_several_pieces(gpu, dtype):
+    """all eight quantities, more than a staging half, as one by one"""
+    ctx = hip.Context(dtype)
+    ctx.set_operator(configs.RECON_UPWIND2, configs.LIM_VANALBADA)
+    ctx.add_patch(73, 75, 77, [0] * 6, (1.0, 1.0, 1.0), [configs.BC_SLIP] * 6, np.zeros((6, configs.NPAR)))
+    ctx.layout()
+    rng = np.random.default_rng(5)
+    n = ctx.patch_cells(0)
+    rho = 1.0 + 0.1 * rng.random(n)
+    vel = 50.0 * rng.standard_normal((3, n))
+    ctx.upload(0, 0, np.stack([rho, *(rho * vel), rho * (2.2e5 + 0.5 * (vel ** 2).sum(0))]).astype(dtype))
+    together = ctx.post_variables(0)
+    for name in ctx.POST_NAMES:
+        assert np.array_equal(together[name], ctx.post_variables(0, (name,))[name]), name
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_pinned_buffers(gpu, dtype):
+    """buffers in pinned memory, which go past the staging memory"""
+    import torch
+
+    ctx = hip.Context(dtype)
+    ctx.set_operator(configs.RECON_UPWIND2, configs.LIM_VANALBADA)
+    shapes = [(3, 1, 1), (5, 7, 9), (33, 35, 37), (80, 81, 83)]
+    for n in shapes:
+        ctx.add_patch(*n, [0] * 6, (1.0, 1.0, 1.0), [configs.BC_SLIP] * 6, np.zeros((6, configs.NPAR)))
+    ctx.layout()
+    rng = np.random.default_rng(6)
+    for p, n in enumerate(shapes):
+        a, b = (torch.empty((5, int(np.prod(n))), pin_memory=True,
+                            dtype=torch.float32 if dtype == np.float32 else torch.float64).numpy() for _ in range(2))
+        U = rng.standard_normal(a.shape).astype(dtype)
+        a[:] = U
+        ctx.upload(p, 0, a)
+        a[:] = 0
+        ctx._chk(ctx.L.drn_patch_download(ctx.h, p, 0, hip._p(b)), "drn_patch_download")
+        assert np.array_equal(b, U), n
+    ctx.close()

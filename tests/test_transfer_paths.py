@@ -1,8 +1,9 @@
 """drn_patch_upload / drn_patch_download / drn_post_variables beyond the pageable
-buffer on one thread: no pinned
+buffer on one thread: buffers that HIP can copy from or to directly, no pinned
 memory left, several threads on one context, and the caller's buffer changed
 right after the call (CPU: k_host_copy is carried out by the stand-in runtime when
 the host waits for it)."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -27,6 +28,16 @@ def _grid(dtype, shapes=SHAPES):
                  for p, n in enumerate(shapes)]
 
 
+def _at(address, like):
+    """an array over the memory at `address`"""
+    buf = (C.c_char * like.nbytes).from_address(address)
+    return np.frombuffer(buf, like.dtype).reshape(like.shape)
+
+
+def _call(ctx, name, p, field, address):
+    ctx._chk(getattr(ctx.L, name)(ctx.h, p, field, C.c_void_p(address)), name)
+
+
 def pageable_child():
     for dtype in (np.float32, np.float64):
         ctx, states = _grid(dtype)
@@ -36,6 +47,24 @@ def pageable_child():
             a[:] = 0
         for p, U in enumerate(states):
             assert np.array_equal(ctx.download(p, 0), U), SHAPES[p]
+        ctx.close()
+
+
+def direct_child():
+    """pinned and device buffers are copied as they are, without staging or helper copies"""
+    for dtype in (np.float32, np.float64):
+        ctx, states = _grid(dtype)
+        for alloc in (fakedev.fake.fake_pinned_alloc, fakedev.fake.fake_device_alloc):
+            for p, U in enumerate(states):
+                a, b = alloc(C.c_size_t(U.nbytes)), alloc(C.c_size_t(U.nbytes))
+                _at(a, U)[:] = U
+                fakedev.clear()
+                _call(ctx, "drn_patch_upload", p, 1, a)
+                _at(a, U)[:] = 0
+                _call(ctx, "drn_patch_download", p, 1, b)
+                assert np.array_equal(_at(b, U), U), SHAPES[p]
+                assert not fakedev.launches("k_host_copy"), SHAPES[p]
+                assert sum(c[1] for c in fakedev.launches("memcpy")) == 2 * U.nbytes
         ctx.close()
 
 
@@ -73,6 +102,6 @@ def threads_child():
         ctx.close()
 
 
-@pytest.mark.parametrize("child", ["pageable_child", "no_pinned_child", "threads_child"])
+@pytest.mark.parametrize("child", ["pageable_child", "direct_child", "no_pinned_child", "threads_child"])
 def test_transfers(tmp_path, child):
     run_child(tmp_path, "test_transfer_paths", child)
