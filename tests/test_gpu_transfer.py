@@ -2,6 +2,8 @@
 pinned staging memory: byte for byte, for value counts that do and do not
 divide into 16-byte lanes, patches below and above a staging half (8 MiB), and
 several patches and fields behind each other."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -69,9 +71,10 @@ def test_post_variables_over_several_pieces(gpu, dtype):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_pinned_buffers(gpu, dtype):
     """buffers in pinned memory, which go past the staging memory"""
-    import torch
-
     ctx = hip.Context(dtype)
+    rt = C.CDLL("libamdhip64.so.7")  # the runtime the library is linked against
+    rt.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    rt.hipHostFree.argtypes = [C.c_void_p]
     ctx.set_operator(configs.RECON_UPWIND2, configs.LIM_VANALBADA)
     shapes = [(3, 1, 1), (5, 7, 9), (33, 35, 37), (80, 81, 83)]
     for n in shapes:
@@ -79,12 +82,14 @@ def test_pinned_buffers(gpu, dtype):
     ctx.layout()
     rng = np.random.default_rng(6)
     for p, n in enumerate(shapes):
-        a, b = (torch.empty((5, int(np.prod(n))), pin_memory=True,
-                            dtype=torch.float32 if dtype == np.float32 else torch.float64).numpy() for _ in range(2))
-        U = rng.standard_normal(a.shape).astype(dtype)
+        U = rng.standard_normal((5, int(np.prod(n)))).astype(dtype)
+        h = C.c_void_p()
+        assert rt.hipHostMalloc(C.byref(h), U.nbytes, 0) == 0
+        a = np.frombuffer((C.c_char * U.nbytes).from_address(h.value), dtype).reshape(U.shape)
         a[:] = U
-        ctx.upload(p, 0, a)
+        ctx._chk(ctx.L.drn_patch_upload(ctx.h, p, 0, h), "drn_patch_upload")
         a[:] = 0
-        ctx._chk(ctx.L.drn_patch_download(ctx.h, p, 0, hip._p(b)), "drn_patch_download")
-        assert np.array_equal(b, U), n
+        ctx._chk(ctx.L.drn_patch_download(ctx.h, p, 0, h), "drn_patch_download")
+        assert np.array_equal(a, U), n
+        rt.hipHostFree(h)
     ctx.close()
