@@ -1228,10 +1228,8 @@ __device__ __forceinline__ T limited_x(T d01, T d12) {
       const T num = dfma(d12, d01, t), den = dfma(d01, d01, t) + T(1e-30);
       return d01 * num * drcp<T, true>(den);
     } else {
-      // (r^2 + r) / (r^2 + 1) * d01 with r = d12 / d, d = nonZero(d01, 1e-10),
-      // numerator and denominator times d^2: one division instead of two
-      const T d = non_zero(d01, T(1e-10));
-      return ((d12 * (d12 + d)) / dfma(d12, d12, d * d)) * d01;
+      const T r = d12 / non_zero(d01, T(1e-10));
+      return (dfma(r, r, r) / dfma(r, r, T(1))) * d01;
     }
   } else {
     return limited<T, LIM, FAST>(d01, d12);
@@ -1258,21 +1256,6 @@ __device__ __forceinline__ void side_states(const T* m, const T* u, const T* p, 
       const T s = limited_x<T, LIM, true>(u[v] - m[v], p[v] - u[v]);
       if constexpr (MINUS) at_minus[v] = dfma(T(-0.5), s, u[v]);
       if constexpr (PLUS) at_plus[v] = dfma(T(0.5), s, u[v]);
-    } else if constexpr (LIM == LIM_VANALBADA) {
-      // The two limited terms, lim(b/a) a and lim(a/b) b, differ only where
-      // nonZero replaces one of two nonzero differences; elsewhere one division,
-      // the first term's, serves both faces.
-      const T a = u[v] - m[v], b = p[v] - u[v];
-      const bool two = (dabs(a) < T(1e-10) || dabs(b) < T(1e-10)) && a != T(0) && b != T(0);
-      T s = T(0);
-      if constexpr (PLUS) {
-        s = limited_x<T, LIM, FAST>(a, b);
-        at_plus[v] = hm ? dfma(T(0.5), s, u[v]) : u[v];
-      }
-      if constexpr (MINUS) {
-        if (!PLUS || two) s = limited_x<T, LIM, FAST>(two ? b : a, two ? a : b);
-        at_minus[v] = hp ? dfma(T(-0.5), s, u[v]) : u[v];
-      }
     } else {
       if constexpr (MINUS) {
         const T s = limited_x<T, LIM, FAST>(u[v] - p[v], m[v] - u[v]);
@@ -1382,14 +1365,13 @@ __device__ __forceinline__ FaceFlux<T> face_flux_x(const T* vl, const T* vr, T A
       const T Tt = e / Gas<T>::CV;
       p = r * Gas<T>::R * Tt;
       a = dsqrt(Gas<T>::GAMMA * Gas<T>::R * Tt);
-      q[3] = (var[4] + p) * ir;
+      q[3] = (var[4] + p) / r;
     };
     prim(vl, rl, al, pl, F.l);
     prim(vr, rr, ar, pr, F.r);
     const T a = T(0.5) * (al + ar);
-    const T ia = T(1) / a;
-    mach_split_x<T, 1>(F.l[DIR], ia, m4l, p5l);
-    mach_split_x<T, -1>(F.r[DIR], ia, m4r, p5r);
+    mach_split_x<T, 1>(F.l[DIR] / a, T(1), m4l, p5l);
+    mach_split_x<T, -1>(F.r[DIR] / a, T(1), m4r, p5r);
     const T M = m4l + m4r;
     F.x = a * A;
     F.y = dfma(rl, M > T(0) ? M : T(0), rr * (M < T(0) ? M : T(0)));
