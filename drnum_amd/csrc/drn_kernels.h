@@ -1374,10 +1374,11 @@ __device__ __forceinline__ FaceFlux<T> face_flux_x(const T* vl, const T* vr, T A
     mach_split_x<T, -1>(F.r[DIR] / a, T(1), m4r, p5r);
     const T M = m4l + m4r;
     F.x = a * A;
-    F.y = dfma(rl, M > T(0) ? M : T(0), rr * (M < T(0) ? M : T(0)));
+    // (x + |x|) / 2 and (x - |x|) / 2, which keep a NaN
+    F.y = dfma(rl, M < T(0) ? T(0) : M, rr * (M > T(0) ? T(0) : M));
     const T f0 = F.x * F.y;
-    F.fl = f0 > T(0) ? f0 : T(0);
-    F.fr = f0 < T(0) ? f0 : T(0);
+    F.fl = f0 < T(0) ? T(0) : f0;
+    F.fr = f0 > T(0) ? T(0) : f0;
     F.pa = A;
     F.ps = dfma(p5l, pl, p5r * pr);
   }

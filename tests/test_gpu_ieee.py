@@ -65,3 +65,33 @@ def test_rounding_error_of_the_residual(gpu, recon, mach, pressure, rough):
     print("rms error", recon, mach, pressure, rough, err[0], err[1] / err[0], flush=True)
     assert np.isfinite(err).all()
     assert (err[1:] <= 1.01 * err[0]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("arith", [hip.DRN_ARITH_IEEE, hip.DRN_ARITH_FAST])
+def test_non_finite_values_spread_as_in_the_cell_kernel(gpu, dtype, arith):
+    """Residuals around single NaN and infinite values and a negative energy: the
+    same values are finite as in choice 11, so that the count of non-finite
+    values that a program watches is the same."""
+    w = configs.sod(n=N)
+    U = flow(0.3, 1.0 / 1.4, 0.0, 5).reshape(5, -1).astype(dtype)
+    n = 0
+    for v in range(5):
+        for x in (np.nan, np.inf, -np.inf):
+            U[v, 37 + 2111 * n] = x
+            n += 1
+    U[4, 37 + 2111 * n] = -1.0
+    gg = solver.GpuGrid(w, dtype)
+    gg.ctx.set_arith(arith)
+    gg.ctx.upload(0, 0, U)
+    gg.ctx.upload(0, 1, np.zeros_like(U))
+    out = []
+    for c in (11, 51, 52):
+        gg.ctx.set_tiling(c)
+        gg.ctx.stage(0, 1, 2, 1.0 / N ** 3)
+        out.append(np.isfinite(gg.ctx.download(0, 2)))
+    gg.close()
+    print("non-finite", dtype.__name__, arith, [int((~o).sum()) for o in out], flush=True)
+    assert not out[0].all()
+    for o in out[1:]:
+        assert np.array_equal(o, out[0])
