@@ -643,6 +643,9 @@ static bool use_box_cells(const drn_ctx* ctx, int kind) {
   return kind == K_CELLZ && (ctx->visc || ctx->flags_on) && ctx->pd_stage != ctx->d_pd;
 }
 
+// whether the stages of the RK step run on the descriptors and lists of the boxes
+static bool rk_boxes(const drn_ctx* ctx) { return ctx->fuse && ctx->d_pd_rk; }
+
 template <typename T>
 static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int launch) {
   const T* src = (const T*)ctx->buf[psrc];
@@ -749,7 +752,7 @@ static int do_stage(drn_ctx* ctx, int psrc, int pbase, int pdst, double factor, 
   hipEvent_t stop;
   timer_begin(ctx, 0, &stop);
   ctx->push_now = push;
-  ctx->pd_stage = rk && ctx->fuse && ctx->d_pd_rk ? ctx->d_pd_rk : ctx->d_pd;
+  ctx->pd_stage = rk && rk_boxes(ctx) ? ctx->d_pd_rk : ctx->d_pd;
   if (ctx->prec == DRN_F32)
     stage_t<float>(ctx, psrc, pbase, pdst, (float)factor, launch);
   else
@@ -2758,7 +2761,8 @@ int drn_num_tilings(void) { return kNumTilings; }
 
 // Times every tiling choice on one stage of the given launch form (field 0 ->
 // field 2 with field 1 as base, which leaves fields 0 and 1 untouched) and keeps
-// the fastest.
+// the fastest.  The stage is the RK step's, unless that is the same for every
+// choice (use_box_cells): then a choice sets the list of drn_stage alone.
 int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
   if (!ctx) return DRN_E_ARG;
   if (!ctx->laid_out) return fail(ctx, DRN_E_STATE, "drn_layout not called");
@@ -2772,12 +2776,15 @@ int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
   int best = drn_get_tiling(ctx, launch);
   float best_ms = 1e30f;
   int rc = DRN_OK;
-  std::vector<std::pair<int, int>> tried;  // (effective kind, list order) already timed as the same
+  std::vector<std::pair<int, int>> tried;  // (effective kind, list) already timed as the same
+  const bool alone = (ctx->visc || ctx->flags_on) && rk_boxes(ctx);
   for (int c = 0; c < kNumTilings && rc == DRN_OK; ++c) {
     const int ek = effective_kind(ctx, c);
     // choices that fall back to the same cell kernel on the same list are one candidate
     if (ek == K_CELLZ || ek == K_CELL || ek == K_XM) {
-      const std::pair<int, int> key(ek, kTilings[c].xcd + 4 * kTilings[c].irange);
+      const bool chains = ek == K_CELLZ && launch == DRN_LAUNCH_BATCHED && ctx->d_tz_chain;
+      const int order = std::min(kTilings[c].xcd, chains ? 2 : 1), planes = ek == K_XM ? kTilings[c].irange : 0;
+      const std::pair<int, int> key(ek, order + 4 * planes);
       bool seen = false;
       for (const auto& t : tried) seen = seen || t == key;
       if (seen) continue;
@@ -2786,9 +2793,9 @@ int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
     if (drn_set_tiling(ctx, launch, c) != DRN_OK) continue;
     // a stage and the exchange after it: the cell kernels fill the fused
     // receivers and leave the exchange less to do
-    const bool push = push_active(ctx, launch);
+    const bool push = !alone && push_active(ctx, launch);
     auto trial = [&]() {
-      int r = do_stage(ctx, ctx->map[0], ctx->map[1], ctx->map[2], 0.0, launch, push, true);
+      int r = do_stage(ctx, ctx->map[0], ctx->map[1], ctx->map[2], 0.0, launch, push, !alone);
       return r ? r : do_exchange(ctx, ctx->map[2], push ? X_PART : X_FULL);
     };
     rc = trial();  // warm-up

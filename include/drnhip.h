@@ -340,7 +340,9 @@ int drn_set_tiling(drn_ctx* ctx, int launch, int choice);
 int drn_get_tiling(const drn_ctx* ctx, int launch);
 /* Time every choice on one stage and the exchange after it, for the launch
  * form, on the current state (the state is not modified), and keep the
- * fastest; writes it to *choice if not NULL. */
+ * fastest; writes it to *choice if not NULL.  The stage is that of drn_rk_step.
+ * With the viscous flux or cell flags on a grid with receivers, drn_rk_step runs
+ * one list whatever the choice; then it is drn_stage's. */
 int drn_autotune(drn_ctx* ctx, int launch, int* choice);
 /* Arithmetic of the flux kernels: IEEE division and square root, or the fast
  * form (hardware reciprocal, single-division van Albada, exact 0/1 for the

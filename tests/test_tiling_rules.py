@@ -1,0 +1,57 @@
+"""The work-list choices as drn_get_tiling, drn_autotune and the launches show them
+(CPU: the launches are recorded, not carried out)."""
+import numpy as np
+import pytest
+
+import fakedev
+from fakedev import run_child
+
+
+def context(w, viscous=None):
+    from drnum_amd import hip, host
+
+    hg = host.HostGrid.from_workload(w, fp64_geometry=True)
+    hg.compute_dependencies(w.periodic)
+    ctx = hip.Context(np.float32)
+    ctx.set_operator(w.recon, w.limiter, w.viscous if viscous is None else viscous)
+    hg.to_device(ctx)
+    hg.upload_exchange(ctx)
+    return hg, ctx
+
+
+def stage_lists(call):
+    """(kernel, work list) of the stage launches of a call, in order"""
+    fakedev.clear()
+    call()
+    return [(c[0], c[3]) for c in fakedev.launches("k_stage")]
+
+
+def autotune_child():
+    """With the viscous or the flagged operator every choice runs the same list inside
+    the RK step: the autotuner times drn_stage's lists, each once."""
+    from drnum_amd import configs
+
+    w = configs.viscous_shear(core=9, blocks=(2, 2, 2))
+    for viscous in (True, False):
+        hg, ctx = context(w, viscous)
+        if not viscous:
+            flags = np.zeros(w.patches[0].cells, np.uint8)
+            flags[::5] = 1
+            ctx.set_cell_flags(0, flags)
+        for launch in (0, 1):
+            np_ = len(w.patches) if launch else 1
+            runs = stage_lists(lambda: ctx.autotune(launch))
+            tried = [tuple(runs[q:q + np_]) for q in range(0, len(runs), np_)]
+            # a warm-up and three timed stages per candidate
+            assert len(tried) % 4 == 0 and all(len(set(tried[q:q + 4])) == 1 for q in range(0, len(tried), 4))
+            lists = tried[::4]
+            assert len(lists) > 1 and len(set(lists)) == len(lists), (viscous, launch, len(lists), len(set(lists)))
+            best = ctx.get_tiling(launch)
+            alone = stage_lists(lambda: ctx.stage(0, 1, 2, 0.0, launch))
+            assert tuple(alone) in lists, (viscous, launch, best)
+        ctx.close()
+
+
+@pytest.mark.parametrize("child", ["autotune_child"])
+def test_choices(tmp_path, child):
+    run_child(tmp_path, "test_tiling_rules", child)
