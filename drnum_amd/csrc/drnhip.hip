@@ -587,6 +587,9 @@ static bool column_capable(const drn_ctx* ctx) {
   return fast && ctx->recon == DRN_RECON_UPWIND2 && (ctx->lim == DRN_LIM_VANALBADA || ctx->lim == DRN_LIM_MINMOD);
 }
 
+// whether the stages of the RK step run on the descriptors and lists of the boxes
+static bool rk_boxes(const drn_ctx* ctx) { return ctx->fuse && ctx->d_pd_rk; }
+
 // The tiling choice of a launch form: the one set or autotuned, else by a rule.
 // The box kernel over four planes per item (52) is the fastest or within 6 % of
 // it on every grid measured from 0.3 to 60 M cells in both precisions (64-patch
@@ -604,8 +607,9 @@ static int tiling_of(const drn_ctx* ctx, int launch) {
   const int set = launch == DRN_LAUNCH_BATCHED ? ctx->tiling : ctx->tiling_pp;
   if (set >= 0) return set;
   const bool fast32 = ctx->prec == DRN_F32 && (ctx->arith < 0 || ctx->arith == DRN_ARITH_FAST);
-  if (launch == DRN_LAUNCH_BATCHED && fast32 && ctx->sweep_waves_all >= 48 * (int64_t)ctx->n_cu) return kSweep8;
-  const int n = (ctx->box_rk[1].n > 0 ? ctx->box_rk : ctx->box)[1].n;
+  const bool boxes = rk_boxes(ctx);
+  if (launch == DRN_LAUNCH_BATCHED && fast32 && boxes && ctx->sweep_waves_all >= 48 * (int64_t)ctx->n_cu) return kSweep8;
+  const int n = (boxes ? ctx->box_rk : ctx->box)[1].n;
   const int np = launch == DRN_LAUNCH_BATCHED ? 1 : std::max(1, (int)ctx->descs.size());
   return n / np < ctx->n_cu ? kBoxOnePlane : kBoxFourPlanes;
 }
@@ -642,9 +646,6 @@ static const drn_ctx::BoxList& box_list(const drn_ctx* ctx, int kind) {
 static bool use_box_cells(const drn_ctx* ctx, int kind) {
   return kind == K_CELLZ && (ctx->visc || ctx->flags_on) && ctx->pd_stage != ctx->d_pd;
 }
-
-// whether the stages of the RK step run on the descriptors and lists of the boxes
-static bool rk_boxes(const drn_ctx* ctx) { return ctx->fuse && ctx->d_pd_rk; }
 
 template <typename T>
 static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int launch) {
@@ -730,8 +731,8 @@ static void stage_t(drn_ctx* ctx, int psrc, int pbase, int pdst, T factor, int l
   }
 }
 
-// The cell kernels (choices of kind K_CELL, K_CELLZ, K_CELLZP, K_XM*) can fill the
-// fused z-face receivers themselves; the other kinds leave them to the exchange.
+// The cell kernels (choices of kind K_CELL, K_CELLZ, K_CELLZP, K_XM*, K_CELLXS*,
+// K_BOX* and K_SWEEP) can fill the fused z-face receivers themselves; the other kinds leave them to the exchange.
 static bool push_kind(int kind) {
   return kind == K_CELL || kind == K_CELLZ || kind == K_CELLZP || kind == K_XM || kind == K_XM8 || kind == K_XM7 ||
          kind == K_XML || kind == K_CELLXS2 || kind == K_CELLXS4 || kind == K_BOX1 || kind == K_BOX4 || kind == K_SWEEP;
@@ -2368,7 +2369,7 @@ int drn_set_exchange_fusion(drn_ctx* ctx, int on) {
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   ctx->fuse = on != 0;
   drop_graph(ctx);
-  return DRN_OK;
+  return ctx->laid_out ? build_march(ctx) : DRN_OK;  // the rule's choice may change with the switch
 }
 
 int drn_exchange_fused_cells(const drn_ctx* ctx, int launch, int64_t* n) {

@@ -183,14 +183,16 @@ int drn_exchange(drn_ctx* ctx, int field);
 /* No counterpart in the reference, whose copyDonorData copies every receiver
  * after the stage.  With fusion on (the default), drn_rk_step and
  * drn_rk_graph_run let the cell stage kernels (the tiling kinds of choices 11,
- * 20, 27, 28, 33, 34, 35) fill part of the exchange themselves: the z-face seek
+ * 20, 27, 28 and 33-53) fill part of the exchange themselves: the z-face seek
  * layers of a patch's x/y core columns, one side at a time, where
  * drn_exchange_commit found that side to be an aligned unit-weight copy of
  * one donor patch.  A donor thread writes 0 + its new value into its receiver
  * (the exchange's own sum), the receiver thread skips its store, and the
  * exchange after the stage runs on the other receivers.  The results are
- * bit-identical to fusion off; drn_stage and drn_exchange never fuse.
- * Switching drops a captured graph. */
+ * bit-identical to fusion off; drn_stage and drn_exchange never fuse.  Off, the
+ * stages of these calls also run on whole patches instead of the boxes of cells
+ * that are no receivers (choices 51-53; 53 runs 52), face functors of receiver
+ * layers included.  Switching drops a captured graph. */
 int drn_set_exchange_fusion(drn_ctx* ctx, int on);
 /* Receivers that the stage kernels of drn_rk_step fill themselves for this
  * launch form (DRN_LAUNCH_*) under the current tiling and fusion switch: 0 when
@@ -334,7 +336,7 @@ int drn_post_variables(drn_ctx* ctx, int field, int patch, int mask, double ref_
  *       on (FP32 fast arithmetic inside drn_rk_step and drn_rk_graph_run, patches
  *       of up to about 195 cells along z; otherwise 52).
  * Until a choice is set or autotuned, a rule on the size of the grid picks 51, 52
- * or 53; drn_get_tiling returns the choice in effect. */
+ * or 53.  drn_get_tiling returns the choice that was set, else the rule's. */
 int drn_num_tilings(void);
 int drn_set_tiling(drn_ctx* ctx, int launch, int choice);
 int drn_get_tiling(const drn_ctx* ctx, int launch);

@@ -52,6 +52,25 @@ def autotune_child():
         ctx.close()
 
 
-@pytest.mark.parametrize("child", ["autotune_child"])
+def fusion_child():
+    """drn_get_tiling answers the choice whose kernel runs, with the exchange fusion on
+    and off (then the RK step runs on whole patches, which the sweep does not)"""
+    from drnum_amd import configs
+
+    w = configs.jet(core=40, blocks=5)
+    names = {51: "k_stage_box<float, 1, 0, true, 1>", 52: "k_stage_box<float, 1, 0, true, 4>",
+             53: "k_stage_sweep<float, 1, 0, true, 168, 4>"}
+    hg, ctx = context(w)
+    seen = []
+    for on in (True, False, True):
+        ctx.set_exchange_fusion(on)
+        kernels = {c[0] for c in stage_lists(lambda: ctx.rk_step(w.dt, w.alpha))}
+        assert kernels == {names[ctx.get_tiling()]}, (on, ctx.get_tiling(), kernels)
+        seen.append(ctx.get_tiling())
+    assert seen == [53, 52, 53], seen
+    ctx.close()
+
+
+@pytest.mark.parametrize("child", ["autotune_child", "fusion_child"])
 def test_choices(tmp_path, child):
     run_child(tmp_path, "test_tiling_rules", child)
