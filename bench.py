@@ -17,9 +17,12 @@ is one RK step over all patches.
   reference_faces the FP32 batched form on the same jet with the other domain
               faces as the reference's JetFlux has them (far-field lateral
               faces, a slip wall at the far end).
-  roofline    stage kernel: algorithmic bytes per launch (10 or 15 values of
-              4 B per stored cell: stage 1 reads U^n only) / average launch time
-              from HIP events on the context stream over the timed region.
+  roofline    stage kernel: algorithmic bytes per launch (the state of every
+              stored cell read, the base state of the cells that the launch
+              advances read from stage 2 on, theirs and the fused receivers'
+              written, 5 values of 4 B each; the box and sweep kernels leave the
+              exchange receivers out) / average launch time from HIP events on
+              the context stream over the timed region.
   valu_roofline the same kernel against its compute ceiling: VALU wave
               instructions per launch (committed rocprofv3 summary) / CUs /
               launch time, against the FP32 VALU issue rate measured by
@@ -81,10 +84,30 @@ def setup(w, dtype, launch_tables=True):
     return hg, ctx
 
 
+def stage_cells(hg, w, tiling, n_fused):
+    """Cells whose state, whose base state and whose new state a stage launch of the
+    RK step cannot do without reading, reading and writing.  The box and sweep
+    kernels (choices from 51 on) and the viscous operator advance the boxes of the
+    cells that are no receivers (the latter their planes and rows) and write the
+    fused receivers; the others advance every stored cell."""
+    if tiling < 51 and not w.viscous:
+        return w.total_cells, w.total_cells, w.total_cells
+    box = 0
+    for p, P in enumerate(w.patches):
+        keep = np.ones((P.ni, P.nj, P.nk), dtype=bool)
+        keep.reshape(-1)[np.asarray(hg.tables(p)["receivers"], dtype=np.int64)] = False
+        n = 1
+        for a in range(2 if w.viscous else 3):
+            at = np.flatnonzero(keep.any(axis=tuple(b for b in range(3) if b != a)))
+            n *= int(at[-1] - at[0] + 1) if at.size else 0
+        box += n * P.nk if w.viscous else n
+    return w.total_cells, box, min(w.total_cells, box if w.viscous else box + n_fused)
+
+
 def stage_bytes_per_step(cells, esize, n_stages):
-    # stage 1 reads U^n once (src == base) and writes 5 values; later stages read src and base
-    vals = 10 + 15 * (n_stages - 1)
-    return cells * vals * esize
+    read, base, written = cells
+    # stage 1 reads U^n once (src == base), later stages read src and base
+    return 5 * esize * (n_stages * (read + written) + (n_stages - 1) * base)
 
 
 def run_form(w, dtype, steps, warmup, launch, label, tiling=None, arith=None):
@@ -97,7 +120,6 @@ def run_form(w, dtype, steps, warmup, launch, label, tiling=None, arith=None):
     esize = np.dtype(dtype).itemsize
     S = len(w.alpha)
     ex_bytes, ls_bytes = exchange_fill_bytes(hg, w, esize)
-    n_fused = 0
     if tiling is None:
         # the library's autotuner picks the stage work-list (i-range, XCD order, kernel) for this form
         tiling = ctx.autotune(launch)
@@ -135,8 +157,12 @@ def run_form(w, dtype, steps, warmup, launch, label, tiling=None, arith=None):
     res = dict(wall=wall, ms_per_step=1e3 * wall / steps, mcups=cells * S * steps / wall / 1e6,
                stage_ms=st_ms, stage_n=st_n, exch_ms=ex_ms, exch_n=ex_n, tiling=tiling,
                exch_bytes=ex_bytes, ls_ms=ls_ms, ls_n=ls_n, ls_bytes=ls_bytes, fused=n_fused)
-    # per launch the stage kernel advances all stored cells once
-    bytes_step = stage_bytes_per_step(cells, esize, S)
+    # with a fill, the exchange of the receivers it touched runs before every stage
+    # and is timed with the exchange after the stage: the mean over both
+    if ls_n > 0 and ex_n > S * steps:
+        n_part = S * steps
+        res["exch_bytes"] = (n_part * ex_bytes + (ex_n - n_part) * touched_bytes(hg, w, esize)) / ex_n
+    bytes_step = stage_bytes_per_step(stage_cells(hg, w, tiling, n_fused), esize, S)
     res["stage_bytes_per_launch"] = bytes_step / S
     if launch == hip.DRN_LAUNCH_BATCHED:
         res["stage_gbs"] = res["stage_bytes_per_launch"] / (st_ms * 1e-3) / 1e9 if st_ms > 0 else 0.0
@@ -210,6 +236,38 @@ def exchange_fill_bytes(hg, w, esize):
                 n_ls += len(hg.ls_cells(p, layer)["cells"])
     ls = n_ls * (8 * (4 + 6 * esize) + 5 * esize + 4 + 3 * esize + 5 * esize + 3 * esize + 5 * esize)
     return ex, ls
+
+
+def touched_receivers(hg, w):
+    """(receivers, donor entries) of the exchange between a level-set fill and the next
+    stage: receivers that the fill writes or whose donors it writes"""
+    filled = []
+    for p, P in enumerate(w.patches):
+        f = np.zeros(P.cells, dtype=bool)
+        for layer in range(w.ls_inner_layers):
+            f[np.asarray(hg.ls_cells(p, layer)["cells"], dtype=np.int64)] = True
+        filled.append(f)
+    n_rec = n_pairs = 0
+    for p, P in enumerate(w.patches):
+        t = hg.tables(p)
+        receiver = np.zeros(P.cells, dtype=bool)
+        receiver[np.asarray(t["receivers"], dtype=np.int64)] = True
+        touched = filled[p].copy()
+        lists = []
+        for dp, nrec, stride, r0, w0 in t["donors"]:
+            rec = np.asarray(t["rec_concat"][r0:r0 + nrec], dtype=np.int64)
+            idx = np.asarray(t["donor_index"][w0:w0 + nrec * stride], dtype=np.int64).reshape(nrec, stride)
+            touched[rec[filled[dp][idx].any(axis=1)]] = True
+            lists.append((rec, stride))
+        touched &= receiver
+        n_rec += int(touched.sum())
+        n_pairs += sum(int(touched[rec].sum()) * stride for rec, stride in lists)
+    return n_rec, n_pairs
+
+
+def touched_bytes(hg, w, esize):
+    n_rec, n_pairs = touched_receivers(hg, w)
+    return n_rec * (4 + 5 * esize) + n_pairs * (4 + 6 * esize)
 
 
 def kernel_roofline(ms, nbytes, traffic=None):
