@@ -5,6 +5,7 @@ import pytest
 
 from drnum_amd import configs, hip, solver
 from oracle import oracle as O
+from test_gpu_parity import make
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +96,30 @@ def test_non_finite_values_spread_as_in_the_cell_kernel(gpu, dtype, arith):
     assert not out[0].all()
     for o in out[1:]:
         assert np.array_equal(o, out[0])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("arith", [hip.DRN_ARITH_IEEE, hip.DRN_ARITH_FAST])
+def test_non_finite_values_after_a_step(gpu, dtype, arith):
+    """The same on patches with exchange receivers after one RK step, for all cells:
+    boxes, and the sweep (53) in FP32 fast arithmetic, beside choice 11"""
+    w = configs.jet(core=24, blocks=2)
+    rng = np.random.default_rng(8)
+    states = [w.initial_state(p, dtype) for p in range(len(w.patches))]
+    for U in states:
+        for v in range(5):
+            U.reshape(5, -1)[v, rng.integers(0, U.reshape(5, -1).shape[1])] = rng.choice([np.nan, np.inf, -np.inf])
+    masks = []
+    for choice in (11, 51, 52, 53):
+        _, gg = make(w, dtype)
+        gg.ctx.set_arith(arith)
+        gg.ctx.set_tiling(choice)
+        gg.upload_state(states)
+        gg.rk_step()
+        masks.append([np.isfinite(U) for U in gg.state(0)])
+        gg.close()
+    print("non-finite after a step", dtype.__name__, arith, [sum(int((~a).sum()) for a in m) for m in masks], flush=True)
+    assert not all(a.all() for a in masks[0])
+    for m in masks[1:]:
+        for a, b in zip(masks[0], m):
+            assert np.array_equal(a, b)
