@@ -23,7 +23,10 @@ namespace {
 
 constexpr int NBUF = 3;
 constexpr int ALIGN_CELLS = 64;
-constexpr int kSweepN4[2] = {168, 328};  // tile sizes of the sweep kernel over 4 and 8 wavefronts
+// Tile sizes of the sweep kernel over 4 and 8 wavefronts, in 16-byte units per
+// variable: rows of up to 101 cells at 5 workgroups of 4 wavefronts per CU, and of up
+// to 199 cells at 2 of 8.  Larger tiles were not tried.
+constexpr int kSweepN4[2] = {168, 328};
 constexpr int kRedBlocksPerCu = 8;  // a full device of 256-thread workgroups
 
 struct ExchangeTables {
@@ -594,10 +597,10 @@ static bool rk_boxes(const drn_ctx* ctx) { return ctx->fuse && ctx->d_pd_rk; }
 // The box kernel over four planes per item (52) is the fastest or within 6 % of
 // it on every grid measured from 0.3 to 60 M cells in both precisions (64-patch
 // jet, FP32: 0.467 ms per stage and exchange against 0.612 of choice 11 and
-// 0.495 of 49; 27-patch jet, FP64: 0.263 against 0.458 of 11), with two
+// 0.495 of 49; 27-patch jet of 3.5 M cells, FP64: 0.294 against 0.421 of 11), with two
 // exceptions.  Where its items would not give every CU one, the one-plane form
 // (51) spreads the cells over four times as many workgroups: 8 patches of 8^3
-// cells, FP64, 14.2 us against 22.7; 8 patches of 16^3, FP32, 160 items, 9.4
+// cells, FP64, 14.2 us per stage against 23.4; 8 patches of 16^3, FP32, 160 items, 9.4
 // against 9.5.  In FP32 fast arithmetic the sweep (53) is faster once its list
 // fills the device (20 wavefronts per CU) about two and a half times, with the
 // state beyond the caches: us per stage and exchange of 52 / 53 on 3.5 M cells
@@ -1165,8 +1168,9 @@ static int do_rk_step(drn_ctx* ctx, double dt, int n_alpha, const double* alpha,
 
 // The functions below were declared extern "C" by drnhip.h and keep C linkage.
 
-// Partial sums of drn_core_sums_noalloc: 5 doubles per plane chunk of the
-// stage work list, at most kScratchChunks chunks (40 MiB on every device the
+// Partial sums of drn_core_sums_noalloc: 5 doubles per workgroup of the
+// reduction.  The size allows one workgroup per plane chunk of the largest grid
+// that the call accepts, kScratchChunks chunks (40 MiB on every device the
 // library runs on, held until the process ends).  In host code `scratch` names
 // a host-side stand-in: kernels and copies take the address that
 // hipGetSymbolAddress gives for the current device, kept per device below.

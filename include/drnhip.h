@@ -241,8 +241,8 @@ int drn_core_sums(drn_ctx* ctx, int field, double* out);
  * memory (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc): drn_core_sums with the result written to d_out, 5 doubles of
  * DEVICE memory that the caller owns, asynchronously on the context stream
- * (drn_sync before reading it).  The per-chunk partial sums go to a fixed
- * device array of the library (40 MiB, held on every device the library runs
+ * (drn_sync before reading it).  The partial sums, 5 doubles per workgroup
+ * (at most 8 workgroups per CU), go to a fixed device array of the library (40 MiB, held on every device the library runs
  * on until the process ends) instead of context memory, so the call allocates
  * nothing.  The sums equal drn_core_sums bit for bit.  At most 2^20 plane
  * chunks of 256 cells (about 2.7e8 stored cells): DRN_E_RANGE above.  Every

@@ -47,6 +47,18 @@ def test_stage_bytes_of_the_viscous_box():
     assert bench().stage_cells(_grid(w), w, 35, 0) == (8 * 1000, n, n)
 
 
+def test_the_default_choice_of_the_jet_has_a_profile():
+    """the traffic and VALU entries of the bench line need the running choice's counters"""
+    b = bench()
+    for choice in (52, 53):
+        row = b.sweep_profile(choice)
+        # no more than twice the bytes that the launch cannot do without
+        assert 0.9e9 < row["traffic"] < 2.0e9 and 1e8 < row["instructions"] < 1e9
+        assert 87_629_568 <= row["exchange"] < 2 * 87_629_568
+    assert b.sweep_profile(11) is None
+    assert b.profile_hash(b.SWEEP_TABLE) is not None
+
+
 def touched_child():
     from drnum_amd import configs, hip
 

@@ -68,6 +68,19 @@ def test_rounding_error_of_the_residual(gpu, recon, mach, pressure, rough):
     assert (err[1:] <= 1.01 * err[0]).all()
 
 
+@pytest.mark.parametrize("power", [30, 45, 52, 60, 84, 110])
+def test_large_states(gpu, power):
+    """FP32 states times a power of two, up to where their squares leave the type's
+    range: the residual is homogeneous of degree one, and with differences that are
+    zero or above nonZero's 1e-10 every value of it scales exactly."""
+    w = configs.sod(n=N)
+    U = flow(0.3, 1.0 / 1.4, 0.3, 9).reshape(5, -1).astype(np.float32)
+    scale = np.float32(2.0) ** power
+    for small, large in zip(residuals(w, U, (51, 52), np.float32), residuals(w, U * scale, (51, 52), np.float32)):
+        assert np.isfinite(large).all()
+        assert np.array_equal(large, small * scale)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("arith", [hip.DRN_ARITH_IEEE, hip.DRN_ARITH_FAST])
 def test_non_finite_values_spread_as_in_the_cell_kernel(gpu, dtype, arith):
