@@ -2786,7 +2786,7 @@ int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
   for (int c = 0; c < kNumTilings && rc == DRN_OK; ++c) {
     const int ek = effective_kind(ctx, c);
     // choices that fall back to the same cell kernel on the same list are one candidate
-    if (ek == K_CELLZ || ek == K_CELL || ek == K_XM) {
+    if (ek == K_CELLZ || ek == K_CELL || ek == K_XM || ek == K_BOX4) {
       const bool chains = ek == K_CELLZ && launch == DRN_LAUNCH_BATCHED && ctx->d_tz_chain;
       const int order = std::min(kTilings[c].xcd, chains ? 2 : 1), planes = ek == K_XM ? kTilings[c].irange : 0;
       const std::pair<int, int> key(ek, order + 4 * planes);
@@ -2796,6 +2796,8 @@ int drn_autotune(drn_ctx* ctx, int launch, int* choice) {
       tried.push_back(key);
     }
     if (drn_set_tiling(ctx, launch, c) != DRN_OK) continue;
+    // without a list of its own the sweep runs the box kernel, which has been timed
+    if (ek == K_SWEEP && (!rk_boxes(ctx) || ctx->sweep[launch == DRN_LAUNCH_BATCHED ? 0 : 1].n == 0)) continue;
     // a stage and the exchange after it: the cell kernels fill the fused
     // receivers and leave the exchange less to do
     const bool push = !alone && push_active(ctx, launch);

@@ -7,12 +7,12 @@ import fakedev
 from fakedev import run_child
 
 
-def context(w, viscous=None):
+def context(w, viscous=None, dtype=np.float32):
     from drnum_amd import hip, host
 
     hg = host.HostGrid.from_workload(w, fp64_geometry=True)
     hg.compute_dependencies(w.periodic)
-    ctx = hip.Context(np.float32)
+    ctx = hip.Context(dtype)
     ctx.set_operator(w.recon, w.limiter, w.viscous if viscous is None else viscous)
     hg.to_device(ctx)
     hg.upload_exchange(ctx)
@@ -52,6 +52,28 @@ def autotune_child():
         ctx.close()
 
 
+def sweep_fallback_child():
+    """Where the sweep does not run (FP64, IEEE, rows too long for its tile, no receivers)
+    it is no candidate beside the box kernel that stands in for it."""
+    from drnum_amd import configs, hip
+
+    long_rows = configs.Workload("rows", configs.block_grid([6, 6, 500], [1, 1, 2], [1.0] * 3, 2, [True] * 3,
+                                                            [configs.BC_SLIP] * 6), configs.RECON_UPWIND2,
+                                 configs.LIM_VANALBADA, [1.0] * 3, [1.0], 1e-3, None)
+    for w, dtype, arith in ((configs.jet(core=9, blocks=2), np.float64, None),
+                            (configs.jet(core=9, blocks=2), np.float32, hip.DRN_ARITH_IEEE),
+                            (long_rows, np.float32, None), (configs.sod(n=16), np.float32, None)):
+        hg, ctx = context(w, dtype=dtype)
+        if arith is not None:
+            ctx.set_arith(arith)
+        for launch in (0, 1):
+            np_ = len(w.patches) if launch else 1
+            runs = [k for k, _ in stage_lists(lambda: ctx.autotune(launch)) if k.startswith("k_stage_box")]
+            # one and four planes per item: a warm-up and three timed stages each
+            assert len(runs) == 2 * 4 * np_ and len(set(runs)) == 2, (w.name, dtype, launch, len(runs), set(runs))
+        ctx.close()
+
+
 def fusion_child():
     """drn_get_tiling answers the choice whose kernel runs, with the exchange fusion on
     and off (then the RK step runs on whole patches, which the sweep does not)"""
@@ -71,6 +93,6 @@ def fusion_child():
     ctx.close()
 
 
-@pytest.mark.parametrize("child", ["autotune_child", "fusion_child"])
+@pytest.mark.parametrize("child", ["autotune_child", "sweep_fallback_child", "fusion_child"])
 def test_choices(tmp_path, child):
     run_child(tmp_path, "test_tiling_rules", child)
