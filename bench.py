@@ -368,6 +368,8 @@ def profile_hash(path):
 def profile_current(path):
     """whether a committed profile summary was taken of the current kernel sources"""
     return profile_hash(path) == kernel_source_hash()
+
+
 VALU_PROBE = os.path.join(ROOT, "drnum_amd", "lib", "valu_probe")
 
 
@@ -386,6 +388,29 @@ def measured_valu_instructions(tiling):
             except ValueError:
                 return None
     return None
+
+
+SWEEP_TABLE = os.path.join(ROOT, "profiles", "stage_sweep_jet4x64_fp32.md")
+
+
+def sweep_profile(tiling):
+    """The committed summary of the box and sweep kernels on this workload: HBM bytes
+    and VALU wave instructions per stage launch of a work-list choice, and HBM bytes
+    of the exchange after it.  None for a choice that it does not hold."""
+    try:
+        lines = open(SWEEP_TABLE).read().splitlines()
+    except OSError:
+        return None
+    out = {}
+    for ln in lines:
+        cols = [c.strip() for c in ln.strip().strip("|").split("|")]
+        if len(cols) != 7:
+            continue
+        if cols[0] == str(tiling) and cols[1].startswith("k_stage"):
+            out["instructions"], out["traffic"] = float(cols[3]), float(cols[6])
+        elif cols[1].startswith("k_exchange_single<float>"):
+            out["exchange"] = float(cols[6])
+    return out if "traffic" in out else None
 
 
 def valu_ceiling():
@@ -574,21 +599,29 @@ def main():
     default_workload = args.workload == "jet" and (args.core, args.blocks) == (64, 4)
     # figures read from committed rocprofv3 summaries hold only for the kernel
     # sources they were taken of: a summary of another build is reported stale
-    traffic_current = profile_current(TRAFFIC_TABLE)
-    valu_current = profile_current(VALU_TABLE)
-    traffic = measured_traffic(f32["tiling"]) if default_workload else None
+    traffic_table, valu_table = TRAFFIC_TABLE, VALU_TABLE
+    traffic = exch_traffic = insts = None
+    if default_workload:
+        sweep = sweep_profile(f32["tiling"])
+        if sweep:
+            traffic_table = valu_table = SWEEP_TABLE
+            traffic, insts, exch_traffic = sweep["traffic"], sweep["instructions"], sweep.get("exchange")
+        else:
+            traffic, insts = measured_traffic(f32["tiling"]), measured_valu_instructions(f32["tiling"])
+            exch_traffic = measured_exchange_traffic()
+    traffic_current = profile_current(traffic_table)
+    valu_current = profile_current(valu_table)
     # compute ceiling of the same kernel: VALU instructions per launch (committed
     # profile of this workload) over the live launch time, against the probe
     valu = None
-    insts = measured_valu_instructions(f32["tiling"]) if default_workload else None
     probe = valu_ceiling() if insts else None
     if insts and probe:
         rate = insts / probe["cus"] / (f32["stage_ms"] * 1e6)
         valu = {"bound": "valu", "achieved": round(rate, 3), "peak": probe["peak"], "unit": "wave-instr/CU/ns",
                 "frac": round(rate / probe["peak"], 4), "instructions_per_launch": insts,
                 "stale": not valu_current,
-                "source": "SQ_INSTS_VALU from profiles/stage_valu_jet4x64_fp32.md (tiling %d); peak measured now by "
-                          "drnum_amd/lib/valu_probe" % f32["tiling"]}
+                "source": "SQ_INSTS_VALU from profiles/%s (tiling %d); peak measured now by "
+                          "drnum_amd/lib/valu_probe" % (os.path.basename(valu_table), f32["tiling"])}
         log("valu", valu)
     out = {
         "metric": METRIC,
@@ -622,8 +655,8 @@ def main():
             "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": traffic if traffic_current else None,
-            "traffic_source": ("rocprofv3 FETCH_SIZE/WRITE_SIZE, profiles/stage_traffic_jet4x64_fp32.md, tiling %d"
-                               % f32["tiling"]) if traffic else None,
+            "traffic_source": ("rocprofv3 FETCH_SIZE/WRITE_SIZE, profiles/%s, tiling %d"
+                               % (os.path.basename(traffic_table), f32["tiling"])) if traffic else None,
             # a summary taken of other kernel sources: its figure, not used as traffic
             "traffic_stale": None if (traffic is None or traffic_current) else traffic,
             "kernel_source_sha256": kernel_source_hash(),
@@ -678,8 +711,7 @@ def main():
         "stage_kernel_ms": round(f32["stage_ms"], 4),
         "exchange_ms": round(f32["exch_ms"], 4),
         "exchange_roofline": kernel_roofline(f32["exch_ms"], f32["exch_bytes"],
-                                             measured_exchange_traffic() if default_workload and traffic_current
-                                             else None),
+                                             exch_traffic if traffic_current else None),
         "exchange_fused_receivers": f32["fused"],
         "levelset_fill_roofline": kernel_roofline(f32["ls_ms"], f32["ls_bytes"]),
         "stream_copy_gbs": round(f32["copy_gbs"], 1),
