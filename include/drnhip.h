@@ -96,8 +96,9 @@ int drn_set_operator(drn_ctx* ctx, int recon, int limiter);
  * to every interior face flux after the Euler flux, as the applications' flux
  * classes compose them (EaFlux::xField, drnumCylinder/main.h:127-163; JetFlux,
  * drnumJetDemo/jetflux.h:100-139); the face functors are unchanged.  Every
- * tiling choice then runs the z-shared cell kernel (27 or 28 by list order).
- * Default 0. */
+ * tiling choice then runs the z-shared cell kernel (27 or 28 by list order); on a
+ * grid with receivers drn_rk_step and drn_rk_graph_run run it on one list, the
+ * planes and rows of the cells that are no receivers.  Default 0. */
 int drn_set_viscous(drn_ctx* ctx, int on);
 
 /* ---- patches ------------------------------------------------------------ */
@@ -112,7 +113,8 @@ int drn_num_patches(const drn_ctx* ctx);
 size_t drn_patch_cells(const drn_ctx* ctx, int id);
 /* Host <-> device copy of one field of one patch (GPU_Patch::copyToDevice /
  * copyFromDevice, gpu_patch.h:131-140; updateDevice/updateHost, gpu_patchiterator.h:85-126).
- * `host` holds 5*N values of the context precision, variable-major. Synchronous. */
+ * `host` holds 5*N values of the context precision, variable-major. Synchronous.
+ * Several threads may hand over patches of one context at once. */
 int drn_patch_upload(drn_ctx* ctx, int id, int field, const void* host);
 int drn_patch_download(drn_ctx* ctx, int id, int field, void* host);
 /* PatchIterator::copyField (patchiterator.h:96-101) for all patches. */
@@ -134,8 +136,8 @@ int drn_swap_fields(drn_ctx* ctx, int a, int b);
  *                      outer neighbour i0 is a split face stays first order
  *                      (upwind2.h:41).
  * While any patch has flags every tiling choice runs the z-shared cell kernel
- * (27 or 28 by list order) with the flag tests.  After drn_layout; drops a
- * captured graph. */
+ * with the flag tests, on the lists of drn_set_viscous.  After drn_layout; drops
+ * a captured graph. */
 enum { DRN_CELL_INACTIVE = 1, DRN_CELL_INSIDE = 2 };
 int drn_set_cell_flags(drn_ctx* ctx, int patch, const uint8_t* flags);
 
@@ -172,7 +174,9 @@ int drn_exchange_set(drn_ctx* ctx, int recv_id, int n_donors, const int32_t* don
  * the diagonal and zeros elsewhere (aligned patches) changes no finite value
  * and is skipped.  Not calling it leaves every donor of the patch aligned. */
 int drn_exchange_set_turn(drn_ctx* ctx, int recv_id, int n_donors, const double* turn);
-/* Upload all tables set so far into the device gather lists.  Fails with
+/* Upload all tables set so far into the device gather lists.  A failed commit
+ * leaves complete lists only: the stages may run on whole patches, and the grid
+ * may be without exchange.  Fails with
  * DRN_E_RANGE when a donor cell is also a receiver cell: the reference fills
  * receivers patch after patch, the device all at once, so such tables would
  * give order-dependent results (the reference's donor search never produces
@@ -223,9 +227,10 @@ int drn_set_levelset_op(drn_ctx* ctx, int op);
  * with coefficients alpha[0..n-1], the exchange after every stage and the
  * level-set fill (if tables are set) as the post operation.  The state is in
  * field 0 before and after; fields 1 and 2 are used as stage storage.  The
- * exchange before a stage is repeated only when a post operation exists or
- * when the state was written since its last exchange (an upload, a copy, a
- * drn_stage or a fill into it); otherwise it would reproduce the same values. */
+ * exchange before a stage is repeated only when the state was written since its
+ * last exchange (an upload, a copy, a drn_stage or a fill into it); otherwise it
+ * would reproduce the same values.  Where a fill alone wrote it, only the
+ * receivers that the fill can have changed are copied. */
 int drn_rk_step(drn_ctx* ctx, double dt, int n_alpha, const double* alpha, int launch);
 /* `n_steps` drn_rk_step calls (batched launch form) replayed from HIP graphs.
  * A graph holds the steps until the field map returns to its start (two for an
